@@ -13,12 +13,15 @@
 // contiguous HBM (a row-major fragment touches 16 rows K*2 bytes apart), which
 // measured 20-25% faster for 16-row activations on MI355X.
 //
-// Kernel: one block per 16-row output tile; KS waves split the K tiles of
-// 128 (4 fragments) into contiguous runs, U tiles in flight per wave, and meet
-// in LDS.  Activations stay row-major; batch rows past B and k past K read
-// as zero through buffer-load range checks.
+// Kernel: one block per 16-column output tile (or three of them, NT) and up to
+// four 16-row activation tiles (MT); KS waves split the K tiles of 128 (4
+// fragments) into contiguous runs, U tiles in flight per wave, and meet in
+// LDS.  Batch rows past B and k past K read as zero through buffer-load range
+// checks.
 #include "tmc_abi.hpp"
 #include "tmc_device.hpp"
+
+#include <cmath>
 
 namespace tmc {
 namespace {
@@ -108,15 +111,24 @@ struct PackedFuseArgs {
 // defaults use 1-4).
 constexpr int kPackedNormWaves = 4;
 
+// Most threads of a block: 16 waves' 128 registers hold every plain form but
+// the two-matrix one over several row tiles; three column tiles take 8 waves.
+constexpr int packed_threads(int mats, int nt, int mt, int fuse) {
+  return nt > 1                ? 512
+         : fuse == kPackedNorm ? kPackedNormWaves * kWave
+         : mats == 2 && mt > 1 ? 512
+                               : 1024;
+}
+
 // ARGMAX (the token-only LM head, emitLMHeadPartialArgmax,
 // DecoderLLMMetalEmitter.cpp:700-728): y is a partial-argmax workspace
 // (argmax_partials, pf.argmax_rows rows of n_out slots); the tile writes,
 // for each batch row, the greatest (value, column) of its 16 logits in the
 // greedy-token order to slot blockIdx.x of that row, and block 0 writes the
 // slot count.  The values are the logits the plain form stores.
-template <int MATS, int U, typename OutT, bool XP = false, bool YP = false, bool ROPE = false,
-          int FUSE = kPackedPlain, bool ARGMAX = false>
-__global__ __launch_bounds__(FUSE == kPackedNorm ? kPackedNormWaves * kWave : 1024) void packed_gemm_kernel(const half_t* __restrict__ x,
+template <int MATS, int NT, int MT, int U, typename OutT, bool XP = false, bool YP = false,
+          bool ROPE = false, int FUSE = kPackedPlain, bool ARGMAX = false>
+__global__ __launch_bounds__(packed_threads(MATS, NT, MT, FUSE)) void packed_gemm_kernel(const half_t* __restrict__ x,
                                                            const half_t* __restrict__ p0,
                                                            const half_t* __restrict__ p1,
                                                            OutT* __restrict__ y, int m_rows,
@@ -127,71 +139,95 @@ __global__ __launch_bounds__(FUSE == kPackedNorm ? kPackedNormWaves * kWave : 10
   static_assert(FUSE != kPackedResidual || (MATS == 1 && !ROPE), "residual: plain projection");
   static_assert(!ARGMAX || (MATS == 1 && !ROPE && !YP && FUSE != kPackedResidual),
                 "the argmax epilogue follows one fp32 projection");
-  extern __shared__ float red[];  // [ks][MATS][4][64], then kPackedNorm: [ks][16] squares
+  // [ks][MATS][MT][4][64], then kPackedNorm: [ks][MT][16] squares
+  extern __shared__ float red[];
   const int lane = threadIdx.x & (kWave - 1);
   const int ks = threadIdx.x / kWave;
   const int j = lane & 15;
   const int g = lane >> 4;
-  const int nt = blockIdx.x;
+  const int nt0 = blockIdx.x * NT;
   const int chunks = (k_in + 31) / 32;
+  const int n_tiles = (n_out + 15) / 16;
   const __amdgpu_buffer_rsrc_t rx =
-      buffer_rsrc(x, XP ? (unsigned)chunks * 1024u : (unsigned)m_rows * (unsigned)k_in * 2u);
+      buffer_rsrc(x, XP ? (unsigned)MT * (unsigned)chunks * 1024u
+                        : (unsigned)m_rows * (unsigned)k_in * 2u);
   const __amdgpu_buffer_rsrc_t r0 = buffer_rsrc(p0, packed_bytes);
   const __amdgpu_buffer_rsrc_t r1 = buffer_rsrc(MATS == 2 ? p1 : p0, packed_bytes);
-  const unsigned x_row = j < m_rows ? (unsigned)j * (unsigned)k_in * 2u : kNone;
-  const unsigned w_base = (unsigned)nt * (unsigned)chunks * 1024u + (unsigned)lane * 16u;
+  int nt = nt0;  // the epilogue's output tile
   // Output element of epilogue item q of this thread (item = threadIdx.x +
-  // q * threads, < 4 * 64): (row, col) and its index in y's layout.
+  // q * threads, < 4 * 64 * MT): (row, col) and its index in y's layout.
   auto item_at = [&](int idx, int& row, int& col) -> size_t {
-    const int l = idx % kWave, r = idx / kWave;
-    row = 4 * (l >> 4) + r;
+    const int l = idx % kWave, r = idx / kWave;  // r: 4 mt + accumulator register
+    row = 16 * (r >> 2) + 4 * (l >> 4) + (r & 3);
     col = nt * 16 + (l & 15);
-    if constexpr (YP)  // pass-relative fragment slot of (row, col)
-      return ((size_t)(col >> 5) * 64 + row + 16 * ((col & 31) >> 3)) * 8 + (col & 7);
+    if constexpr (YP)  // fragment slot of (row, col): its 16-row pass, then within the pass
+      return (size_t)(row >> 4) * ((n_out + 31) / 32) * 512 +
+             ((size_t)(col >> 5) * 64 + (row & 15) + 16 * ((col & 31) >> 3)) * 8 + (col & 7);
     return (size_t)row * n_out + col;
   };
   // kPackedResidual: the residual of each epilogue item is loaded first, ahead
   // of the weight stream, so the epilogue waits on no memory (at batch 16 the
   // o and down projections run one block per CU and end together, so a load
   // in the epilogue was a round trip at the end of every launch)
-  constexpr int kItems = 4;  // epilogue items per thread at one wave per tile
+  constexpr int kItems = 4 * MT;  // epilogue items per thread at one wave per tile
   half_t res_pre[kItems];
   if constexpr (FUSE == kPackedResidual) {
 #pragma unroll
     for (int q = 0; q < kItems; ++q) {
       const int idx = (int)threadIdx.x + q * ks_count * kWave;
       int row, col;
-      const size_t at = item_at(idx < 4 * kWave ? idx : 0, row, col);
-      res_pre[q] = idx < 4 * kWave && row < m_rows && col < n_out ? pf.residual[at] : half_t(0.0f);
+      const size_t at = item_at(idx < kItems * kWave ? idx : 0, row, col);
+      res_pre[q] = idx < kItems * kWave && row < m_rows && col < n_out ? pf.residual[at] : half_t(0.0f);
     }
   }
-  float squares = 0.0f;  // kPackedNorm: row j's sum of squares over this lane's k
-  f4 acc[MATS];
+  float squares[MT];  // kPackedNorm: row 16 mt + j's sum of squares over this lane's k
+  f4 acc[MATS][NT][MT];
 #pragma unroll
-  for (int m = 0; m < MATS; ++m) acc[m] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int mt = 0; mt < MT; ++mt) {
+    squares[mt] = 0.0f;
+#pragma unroll
+    for (int m = 0; m < MATS; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[m][t][mt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  // a step is S fragments of 32 k; a wave's run is whole tiles of 128 k
+  constexpr int S = NT > 1 ? 2 : 4;
   const int tiles = (chunks + 3) / 4;
   const int per_wave = (tiles + ks_count - 1) / ks_count;
-  const int first = ks * per_wave;
-  const int last = min(tiles, first + per_wave);
-  for (int t0 = first; t0 < last; t0 += U) {
-    h8 xv[U][4], wv[U][MATS][4];
+  const int first = 4 * ks * per_wave;
+  const int last = min(4 * tiles, first + 4 * per_wave);
+  for (int c0 = first; c0 < last; c0 += U * S) {
+    h8 xv[U][MT][S], wv[U][MATS][NT][S];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int c = (t0 + u) * 4 + s;
-        const bool live = t0 + u < last && c < chunks;
-        const unsigned w_off = live ? w_base + (unsigned)c * 1024u : kNone;
-        wv[u][0][s] = buffer_load16_stream(r0, w_off);
-        if constexpr (MATS == 2) wv[u][1][s] = buffer_load16_stream(r1, w_off);
+      for (int s = 0; s < S; ++s) {
+        const int c = c0 + u * S + s;
+        const bool live = c < last && c < chunks;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const unsigned w_off = live && (NT == 1 || nt0 + t < n_tiles)
+                                     ? ((unsigned)(nt0 + t) * (unsigned)chunks + (unsigned)c) * 1024u +
+                                           (unsigned)lane * 16u
+                                     : kNone;
+          wv[u][0][t][s] = buffer_load16_stream(r0, w_off);
+          if constexpr (MATS == 2) wv[u][1][t][s] = buffer_load16_stream(r1, w_off);
+        }
         const int kk = c * 32 + 8 * g;
-        if constexpr (XP)  // rows past the batch are never read (their slots are unset)
-          xv[u][s] = buffer_load16(
-              rx, live && kk < k_in && j < m_rows ? ((unsigned)c * 64u + (unsigned)lane) * 16u
-                                                  : kNone);
-        else
-          xv[u][s] = buffer_load16(
-              rx, live && kk < k_in && x_row != kNone ? x_row + (unsigned)kk * 2u : kNone);
+        // rows past the batch are never read (XP: their slots are unset)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          const bool in = live && kk < k_in && 16 * mt + j < m_rows;
+          if constexpr (XP)
+            xv[u][mt][s] = buffer_load16(
+                rx, in ? ((unsigned)(mt * chunks + c) * 64u + (unsigned)lane) * 16u : kNone);
+          else
+            xv[u][mt][s] = buffer_load16(
+                rx, in ? (unsigned)(16 * mt + j) * (unsigned)k_in * 2u + (unsigned)kk * 2u : kNone);
+        }
+        // one 16-row tile: the loads stay in this order, weights first
+        // (grouped by the scheduler: o 8.4 -> 9.0 us at 16 rows)
+        if constexpr (MT == 1 && U <= 2) __builtin_amdgcn_sched_barrier(0);
       }
     if constexpr (FUSE == kPackedNorm) {
       // every load of the step goes out before the squares (left to itself
@@ -200,21 +236,32 @@ __global__ __launch_bounds__(FUSE == kPackedNorm ? kPackedNormWaves * kWave : 10
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) squares = dot8(xv[u][s], xv[u][s], squares);
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            squares[mt] = dot8(xv[u][mt][s], xv[u][mt][s], squares[mt]);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < S; ++s)
 #pragma unroll
-        for (int m = 0; m < MATS; ++m)
-          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[u][s], wv[u][m][s], acc[m], 0, 0, 0);
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int m = 0; m < MATS; ++m)
+              acc[m][t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  xv[u][mt][s], wv[u][m][t][s], acc[m][t][mt], 0, 0, 0);
   }
-  float* red_sq = red + ks_count * MATS * 4 * kWave;
+  float* red_sq = red + ks_count * MATS * MT * 4 * kWave;
   if constexpr (FUSE == kPackedNorm) {
-    squares += __shfl_xor(squares, 16, kWave);
-    squares += __shfl_xor(squares, 32, kWave);
-    if (g == 0) red_sq[ks * 16 + j] = squares;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      squares[mt] += __shfl_xor(squares[mt], 16, kWave);
+      squares[mt] += __shfl_xor(squares[mt], 32, kWave);
+      if (g == 0) red_sq[(ks * MT + mt) * 16 + j] = squares[mt];
+    }
   }
   // kPackedNorm: 1 / rms of batch row `row` (its waves' squares in order)
   auto row_scale = [&](int row) -> float {
@@ -222,87 +269,97 @@ __global__ __launch_bounds__(FUSE == kPackedNorm ? kPackedNormWaves * kWave : 10
       return 1.0f;
     } else {
       float total = 0.0f;
-      for (int w = 0; w < ks_count; ++w) total += red_sq[w * 16 + row];
+      for (int w = 0; w < ks_count; ++w) total += red_sq[w * 16 * MT + row];
       return 1.0f / sqrtf(total / (float)k_in + pf.eps);
     }
   };
+  // one output tile after the other through the same LDS
 #pragma unroll
-  for (int m = 0; m < MATS; ++m)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[((ks * MATS + m) * 4 + r) * kWave + lane] = acc[m][r];
-  __syncthreads();
-  if constexpr (ROPE) {
-    // 16 batch rows x 8 column pairs of the tile; the pair's even column sits
-    // in lane 16g + 2p and the odd one in the next lane
-    for (int idx = threadIdx.x; idx < 128; idx += ks_count * kWave) {
-      const int p = idx & 7, row = idx >> 3;
-      const int l = 16 * (row >> 2) + 2 * p, r = row & 3;
-      float even = 0.0f, odd = 0.0f;
-      for (int w = 0; w < ks_count; ++w) {
-        even += red[(w * 4 + r) * kWave + l];
-        odd += red[(w * 4 + r) * kWave + l + 1];
-      }
-      const int col = nt * 16 + 2 * p;
-      const float scale = row_scale(row);
-      if (row < m_rows && col < n_out)
-        rope_append_pair(ra, ra.request_base + row, col, even * scale, odd * scale);
-    }
-    return;
-  }
-  if constexpr (ARGMAX) {
-    __shared__ float arg_v[16][16];
-    __shared__ int arg_i[16][16];
-    for (int idx = threadIdx.x; idx < 4 * kWave; idx += ks_count * kWave) {
-      const int l = idx % kWave, r = idx / kWave;
-      float a = 0.0f;
-      for (int w = 0; w < ks_count; ++w) a += red[(w * 4 + r) * kWave + l];
-      const int row = 4 * (l >> 4) + r;
-      const int col = nt * 16 + (l & 15);
-      arg_v[row][l & 15] = col < n_out ? from_float<OutT>(a * row_scale(row)) : -INFINITY;
-      arg_i[row][l & 15] = col < n_out ? col : -1;
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < 16 && (int)threadIdx.x < m_rows) {
-      const int row = threadIdx.x;
-      float best = -INFINITY;
-      int selected = -1;
-      for (int c = 0; c < 16; ++c)
-        if (argmax_better(arg_v[row][c], arg_i[row][c], best, selected)) {
-          best = arg_v[row][c];
-          selected = arg_i[row][c];
-        }
-      const ArgmaxPartials out = argmax_partials(y, pf.argmax_rows, n_out);
-      const size_t at = (size_t)(ra.request_base + row) * n_out + blockIdx.x;
-      out.values[at] = best;
-      out.indices[at] = selected;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0 && ra.request_base == 0) {
-      const ArgmaxPartials out = argmax_partials(y, pf.argmax_rows, n_out);
-      *out.count = (int)gridDim.x;
-    }
-    return;
-  }
-  // acc[r] of lane (j, g) = out[batch 4g + r][row 16nt + j]
-#pragma unroll
-  for (int q = 0; q < kItems; ++q) {
-    const int idx = (int)threadIdx.x + q * ks_count * kWave;
-    if (idx >= 4 * kWave) break;
-    const int l = idx % kWave, r = idx / kWave;
-    float a[2] = {0.0f, 0.0f};
+  for (int t = 0; t < NT; ++t) {
+    nt = nt0 + t;
+    if (NT > 1 && nt >= n_tiles) break;  // block-uniform
+    if (t > 0) __syncthreads();          // the previous tile's sums are read
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
-      for (int w = 0; w < ks_count; ++w) a[m] += red[((w * MATS + m) * 4 + r) * kWave + l];
-    int row, col;
-    const size_t at = item_at(idx, row, col);
-    if (row < m_rows && col < n_out) {
-      const float scale = row_scale(row);
-      if constexpr (MATS == 2)
-        y[at] = gated_value(a[0] * scale, a[1] * scale);
-      else if constexpr (FUSE == kPackedResidual)
-        y[at] = from_float<OutT>(to_float<half_t>(res_pre[q]) +
-                                 to_float<half_t>(from_float<half_t>(a[0])));
-      else
-        y[at] = from_float<OutT>(a[0] * scale);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          red[((ks * MATS + m) * kItems + 4 * mt + r) * kWave + lane] = acc[m][t][mt][r];
+    __syncthreads();
+    if constexpr (ROPE) {
+      // 16 MT batch rows x 8 column pairs of the tile; the pair's even column
+      // sits in lane 16g + 2p and the odd one in the next lane
+      for (int idx = threadIdx.x; idx < 128 * MT; idx += ks_count * kWave) {
+        const int p = idx & 7, row = idx >> 3;
+        const int l = 16 * ((row & 15) >> 2) + 2 * p, r = 4 * (row >> 4) + (row & 3);
+        float even = 0.0f, odd = 0.0f;
+        for (int w = 0; w < ks_count; ++w) {
+          even += red[(w * kItems + r) * kWave + l];
+          odd += red[(w * kItems + r) * kWave + l + 1];
+        }
+        const int col = nt * 16 + 2 * p;
+        const float scale = row_scale(row);
+        if (row < m_rows && col < n_out)
+          rope_append_pair(ra, ra.request_base + row, col, even * scale, odd * scale);
+      }
+      continue;
+    }
+    if constexpr (ARGMAX) {
+      __shared__ float arg_v[16 * MT][16];
+      __shared__ int arg_i[16 * MT][16];
+      for (int idx = threadIdx.x; idx < kItems * kWave; idx += ks_count * kWave) {
+        const int l = idx % kWave, r = idx / kWave;
+        float a = 0.0f;
+        for (int w = 0; w < ks_count; ++w) a += red[(w * kItems + r) * kWave + l];
+        const int row = 16 * (r >> 2) + 4 * (l >> 4) + (r & 3);
+        const int col = nt * 16 + (l & 15);
+        arg_v[row][l & 15] = col < n_out ? from_float<OutT>(a * row_scale(row)) : -INFINITY;
+        arg_i[row][l & 15] = col < n_out ? col : -1;
+      }
+      __syncthreads();
+      if ((int)threadIdx.x < 16 * MT && (int)threadIdx.x < m_rows) {
+        const int row = threadIdx.x;
+        float best = -INFINITY;
+        int selected = -1;
+        for (int c = 0; c < 16; ++c)
+          if (argmax_better(arg_v[row][c], arg_i[row][c], best, selected)) {
+            best = arg_v[row][c];
+            selected = arg_i[row][c];
+          }
+        const ArgmaxPartials out = argmax_partials(y, pf.argmax_rows, n_out);
+        const size_t at = (size_t)(ra.request_base + row) * n_out + nt;
+        out.values[at] = best;
+        out.indices[at] = selected;
+      }
+      if (blockIdx.x == 0 && threadIdx.x == 0 && ra.request_base == 0) {
+        const ArgmaxPartials out = argmax_partials(y, pf.argmax_rows, n_out);
+        *out.count = n_tiles;
+      }
+      continue;
+    }
+    // acc[mt][r] of lane (j, g) = out[batch 16mt + 4g + r][row 16nt + j]
+#pragma unroll
+    for (int q = 0; q < kItems; ++q) {
+      const int idx = (int)threadIdx.x + q * ks_count * kWave;
+      if (idx >= kItems * kWave) break;
+      const int l = idx % kWave, r = idx / kWave;
+      float a[2] = {0.0f, 0.0f};
+#pragma unroll
+      for (int m = 0; m < MATS; ++m)
+        for (int w = 0; w < ks_count; ++w) a[m] += red[((w * MATS + m) * kItems + r) * kWave + l];
+      int row, col;
+      const size_t at = item_at(idx, row, col);
+      if (row < m_rows && col < n_out) {
+        const float scale = row_scale(row);
+        if constexpr (MATS == 2)
+          y[at] = gated_value(a[0] * scale, a[1] * scale);
+        else if constexpr (FUSE == kPackedResidual)
+          y[at] = from_float<OutT>(to_float<half_t>(res_pre[q]) +
+                                   to_float<half_t>(from_float<half_t>(a[0])));
+        else
+          y[at] = from_float<OutT>(a[0] * scale);
+      }
     }
   }
 }
@@ -337,37 +394,76 @@ void default_packed(int64_t batch, int64_t n, int mats, int& unroll, int& ks) {
 // 4 tiles in flight without spills.
 int lm_head_unroll(int64_t batch) { return batch > 8 ? 1 : 4; }
 
+// 16-row activation tiles of one launch.  Batches above 16 read every weight
+// once for up to 64 rows instead of once per 16 (MI355X, 7B widths, 64 rows,
+// packed activations, weights beyond the caches: gate/up 121 -> 44 us, q.k.v
+// 73 -> 34, down 69 -> 30, o 31 -> 13, against floors of 28, 16, 14 and 6).
+// What bounds a launch from there is not HBM but the activation fragments,
+// which every output tile re-reads from L2 (about 15 TB/s over the chip).
+// The two-matrix form holds at most 8 waves' partial sums in 64 KiB of LDS.
+int row_tiles(int64_t batch, int64_t k, int mats, int ks) {
+  const int64_t mt = std::min<int64_t>(4, (batch + 15) / 16);
+  const bool fits = (uint64_t)64 * ((k + 31) / 32 * 32) * 2 < kNone && (mats == 1 || ks <= 8);
+  return fits ? (int)mt : 1;
+}
+
+// 16-column output tiles per block, 1 or 3, above 16 batch rows: three tiles
+// share each activation fragment, and their blocks (8 waves) take one round of
+// the 256 CUs where single tiles (many small blocks) even out over it.  Costs
+// in fragment reads per CU; single tiles win back a quarter by running
+// several blocks per CU.  Measured at K 4096, 24 / 48 / 64 rows, one tile
+// against three: q.k.v (768 tiles) 21.6 / 29.7 / 34.0 against 20.1 / 22.6 /
+// 24.4 us, gate/up (688 pairs) 34.3 / 40.2 / 44.3 against 32.3 / 35.8 / 38.5,
+// LM head (2000) 51 / 71 / 85 against 46 / 55 / 60; two or four tiles were
+// slower than three on each.
+int column_tiles(int mt, int64_t n, int mats) {
+  if (mt == 1) return 1;
+  const double tiles = (double)((n + 15) / 16);
+  const double one = tiles / 256.0 * (mt + mats);
+  const double three = std::ceil(tiles / 3.0 / 256.0) * (mt + 3 * mats);
+  return three < 0.75 * one ? 3 : 1;
+}
+
 template <int MATS, typename OutT, bool XP, bool YP, bool ROPE = false, int FUSE = kPackedPlain,
           bool ARGMAX = false>
 int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int64_t batch,
                int64_t k, int64_t n, int unroll, int ks, hipStream_t st,
                const RopeArgs& rope = RopeArgs{}, const PackedFuseArgs& fuse = PackedFuseArgs{}) {
   const int64_t bytes = packed_elements(n, k) * 2;
-  const dim3 grid((unsigned)((n + 15) / 16));
-  const size_t lds = (size_t)ks * MATS * 4 * kWave * sizeof(float) +
-                     (FUSE == kPackedNorm ? (size_t)ks * 16 * sizeof(float) : 0);
   const int64_t x_pass = XP ? ((k + 31) / 32) * 512 : 16 * k;  // elements per 16-row pass
   const int64_t y_pass = YP ? ((n + 31) / 32) * 512 : 16 * n;
-  for (int64_t r0 = 0; r0 < batch; r0 += 16) {
-    const int rows = (int)std::min<int64_t>(16, batch - r0);
+  const int tiles = row_tiles(batch, k, MATS, ks);
+  for (int64_t r0 = 0; r0 < batch; r0 += 16 * tiles) {
+    const int rows = (int)std::min<int64_t>(16 * tiles, batch - r0);
+    const int mt = (rows + 15) / 16;
+    const int nt = FUSE == kPackedResidual ? 1 : column_tiles(mt, n, MATS);
+    if (nt > 1) ks = 8;
+    const dim3 grid((unsigned)(((n + 15) / 16 + nt - 1) / nt));
+    const size_t lds = (size_t)ks * MATS * mt * 4 * kWave * sizeof(float) +
+                       (FUSE == kPackedNorm ? (size_t)ks * mt * 16 * sizeof(float) : 0);
     const half_t* xs = x + (r0 / 16) * x_pass;
     OutT* ys = ROPE || ARGMAX ? y : y + (r0 / 16) * y_pass;
     RopeArgs ra = rope;
     ra.request_base = (int)r0;
     PackedFuseArgs pf = fuse;
     if (FUSE == kPackedResidual) pf.residual = fuse.residual + (r0 / 16) * y_pass;
-    if (unroll == 1)
-      hipLaunchKernelGGL((packed_gemm_kernel<MATS, 1, OutT, XP, YP, ROPE, FUSE, ARGMAX>), grid,
-                         dim3(ks * kWave), lds, st, xs, p0, p1, ys, rows, (int)n, (int)k, ks,
-                         (unsigned)bytes, ra, pf);
-    else if (unroll == 2)
-      hipLaunchKernelGGL((packed_gemm_kernel<MATS, 2, OutT, XP, YP, ROPE, FUSE, ARGMAX>), grid,
-                         dim3(ks * kWave), lds, st, xs, p0, p1, ys, rows, (int)n, (int)k, ks,
-                         (unsigned)bytes, ra, pf);
-    else
-      hipLaunchKernelGGL((packed_gemm_kernel<MATS, 4, OutT, XP, YP, ROPE, FUSE, ARGMAX>), grid,
-                         dim3(ks * kWave), lds, st, xs, p0, p1, ys, rows, (int)n, (int)k, ks,
-                         (unsigned)bytes, ra, pf);
+#define TMC_PACKED_LAUNCH(N, M, U)                                                               \
+  hipLaunchKernelGGL((packed_gemm_kernel<MATS, N, M, U, OutT, XP, YP, ROPE, FUSE, ARGMAX>), grid,   \
+                     dim3(ks * kWave), lds, st, xs, p0, p1, ys, rows, (int)n, (int)k, ks,        \
+                     (unsigned)bytes, ra, pf)
+    if (nt == 3) {
+      if constexpr (FUSE != kPackedResidual) {
+        if (mt == 4) TMC_PACKED_LAUNCH(3, 4, 1);
+        else if (mt == 3) TMC_PACKED_LAUNCH(3, 3, 1);
+        else TMC_PACKED_LAUNCH(3, 2, 1);
+      }
+    } else if (mt == 4) TMC_PACKED_LAUNCH(1, 4, 1);
+    else if (mt == 3) TMC_PACKED_LAUNCH(1, 3, 1);
+    else if (mt == 2) TMC_PACKED_LAUNCH(1, 2, 2);
+    else if (unroll == 1) TMC_PACKED_LAUNCH(1, 1, 1);
+    else if (unroll == 2) TMC_PACKED_LAUNCH(1, 1, 2);
+    else TMC_PACKED_LAUNCH(1, 1, 4);
+#undef TMC_PACKED_LAUNCH
     if (check_launch("packed_gemm_kernel")) return 1;
   }
   return 0;

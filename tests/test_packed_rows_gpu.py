@@ -1,0 +1,131 @@
+"""Packed GEMMs above 16 batch rows: one launch reads every weight for up to
+64 rows (16-row tiles), and wide outputs share activation fragments between
+three 16-column tiles.  Batches at the edges of the row tiles, widths at the
+edges of the column tiles, K with a ragged tail."""
+import numpy as np
+import pytest
+
+from tests.helpers import assert_f16_path, assert_f32_rel, bits, dev_f16, normal, uniform, values
+
+pytestmark = pytest.mark.gpu
+
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    return t
+
+
+BATCHES = [17, 32, 33, 48, 49, 64, 65]
+
+
+def _rows(tmc, torch, x, packed, b, k, n, layout, cfg, residual=None):
+    xin = tmc.pack_activations(x) if layout else x
+    if residual is None:
+        y = torch.full((b, n), float("nan"), dtype=torch.float32, device="cuda")
+        tmc.gemm_packed_ex(xin, packed, y, b, k, n, layout, cfg)
+    else:
+        y = torch.full((b, n), float("nan"), dtype=torch.float16, device="cuda")
+        tmc.gemm_packed_residual(xin, packed, residual, y, b, k, n, layout, cfg)
+    return y
+
+
+@pytest.mark.parametrize("batch", BATCHES)
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("k,n,ks", [(1160, 200, 4), (2048, 520, 16)])
+def test_row_tiles_equal_single_passes(tmc, orc, torch, batch, layout, k, n, ks):
+    """The same k split gives each row the bits of a launch of its own 16
+    rows: fp32 output and fp16 output with the residual."""
+    cfg = tmc.GemvConfig(3, 1, 1, ks)
+    x = dev_f16(orc.f16(normal(2001 + batch, (batch, k))))
+    packed = tmc.pack_weights(dev_f16(orc.f16(normal(2002, (n, k), 0.02))))
+    res = dev_f16(orc.f16(normal(2003, (batch, n))))
+    for r in (None, res):
+        got = _rows(tmc, torch, x, packed, batch, k, n, layout, cfg, r)
+        want = torch.cat([
+            _rows(tmc, torch, x[a:a + 16].contiguous(), packed, min(16, batch - a), k, n, layout,
+                  cfg, None if r is None else r[a:a + 16].contiguous())
+            for a in range(0, batch, 16)])
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("batch,n", [(17, 12288), (33, 8208), (49, 8217), (64, 12300)])
+def test_three_column_tiles_match_fp64(tmc, orc, torch, batch, n):
+    """Wide outputs (three 16-column tiles per block, the last block short):
+    the fp32 projection within the fp32 rule of 64-bit sums of the same fp16
+    products, and the token-only LM head's tokens from the same logits."""
+    k = 1184
+    x = dev_f16(orc.f16(normal(2011 + batch, (batch, k))))
+    gamma = dev_f16(orc.f16(uniform(2012, (k,), 0.5, 1.5)))
+    w = dev_f16(orc.f16(normal(2013, (n, k), 0.02)))
+    packed = tmc.pack_weights(w)
+    y = _rows(tmc, torch, x, packed, batch, k, n, 1, None)
+    ref = x.double() @ w.double().t()
+    assert_f32_rel(values(y), ref.cpu().numpy(), what=f"b{batch} n{n}")
+    scaled = tmc.pack_weights(w, gamma=gamma)
+    logits = torch.full((batch, n), float("nan"), dtype=torch.float32, device="cuda")
+    xin = tmc.pack_activations(x)
+    tmc.gemm_packed_norm(xin, scaled, logits, batch, k, n, 1e-6, 1)
+    xd = x.double()
+    norm = xd / torch.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
+    ref = norm @ (w.float() * gamma.float()).half().double().t()
+    assert_f32_rel(values(logits), ref.cpu().numpy(), what=f"norm b{batch} n{n}")
+    ws = torch.zeros(tmc.lm_head_argmax_workspace_bytes(batch, n) // 4, dtype=torch.float32,
+                     device="cuda")
+    tok = torch.full((batch,), -7, dtype=torch.int32, device="cuda")
+    tmc.lm_head_argmax_packed_norm(xin, scaled, ws, tok, batch, k, n, 1e-6, 1)
+    assert torch.equal(tok.long(), logits.argmax(-1))
+
+
+@pytest.mark.parametrize("batch,n", [(17, 8216), (40, 200), (63, 8216), (65, 8200)])
+def test_gated_rows_match_fp64(tmc, orc, torch, batch, n):
+    """Gate/up + SiLU*Mul with the folded norm, packed output, at one and
+    three tile pairs per block."""
+    k = 1184
+    x = dev_f16(orc.f16(normal(2021 + batch, (batch, k))))
+    one = dev_f16(orc.f16(np.ones(k, np.float32)))
+    wg = dev_f16(orc.f16(normal(2022, (n, k), 0.02)))
+    wu = dev_f16(orc.f16(normal(2023, (n, k), 0.02)))
+    out = torch.zeros(tmc.packed_activation_elements(batch, n), dtype=torch.float16, device="cuda")
+    tmc.gate_up_silu_packed_norm(tmc.pack_activations(x), tmc.pack_weights(wg, gamma=one),
+                                 tmc.pack_weights(wu, gamma=one), out, batch, k, n, 1e-6, 3)
+    got = torch.empty((batch, n), dtype=torch.float16, device="cuda")
+    tmc.pack_activations(out, got, unpack=True, rows=batch, cols=n)
+    xd = x.double()
+    norm = xd / torch.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
+    g, u = norm @ wg.double().t(), norm @ wu.double().t()
+    assert_f16_path(values(got), (g / (1 + torch.exp(-g)) * u).cpu().numpy(), what=f"b{batch}")
+
+
+@pytest.mark.parametrize("batch,qh", [(33, 8), (64, 48)])
+def test_qkv_rope_rows_equal_unfused(tmc, orc, torch, batch, qh):
+    """RoPE + append in the epilogue of several row (and column) tiles writes
+    the bits of the packed GEMM followed by the append kernel."""
+    kvh, d, hidden, cap, p = qh, 64, 512, 64, 16
+    mp, width = cap // p, 3 * qh * 64
+    rng = np.random.default_rng(2031)
+    w = tmc.pack_weights(dev_f16(orc.f16(normal(2032, (width, hidden), 0.05))))
+    x = tmc.pack_activations(dev_f16(orc.f16(normal(2033, (batch, hidden)))))
+    i32 = lambda a: torch.tensor(np.asarray(a, np.int32), device="cuda")  # noqa: E731
+    ang = np.arange(cap)[:, None] * 10000.0 ** (-np.arange(0, d, 2) / d)
+    cos, sin = (torch.tensor(f(ang).astype(np.float32), device="cuda") for f in (np.cos, np.sin))
+    tables = rng.permutation(batch * mp).reshape(batch, mp)
+    args = (cos, sin, i32(rng.integers(1, cap + 1, batch)), i32(tables), i32([batch]))
+    out = []
+    for fused in (True, False):
+        q = torch.full((batch, qh * d), float("nan"), dtype=torch.float16, device="cuda")
+        kp = torch.zeros((batch * mp, kvh, p, d), dtype=torch.float16, device="cuda")
+        vp = torch.zeros_like(kp)
+        if fused:
+            tmc.qkv_rope_append_packed(x, w, *args, q, kp, vp, batch, hidden, qh, kvh, d, cap, p,
+                                       mp, 1)
+        else:
+            qkv = torch.empty((batch, width), dtype=torch.float16, device="cuda")
+            tmc.gemm_packed_ex(x, w, qkv, batch, hidden, width, 1)
+            tmc.decode_rope_append(qkv, *args, q, kp, vp, batch, qh, kvh, d, cap, p, mp)
+        torch.cuda.synchronize()
+        out.append([bits(t) for t in (q, kp, vp)])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
