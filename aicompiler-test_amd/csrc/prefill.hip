@@ -72,7 +72,7 @@ struct PaBlockRegs {
 // position is at or past `end` or its page is absent).  BUF (pools below
 // 4 GiB): raw buffer loads with the out-of-range offset for absent data, so
 // every load issues unconditionally; otherwise predicated global loads.
-template <int D, bool BUF, bool OFFS>
+template <int D, bool BUF>
 __device__ __forceinline__ void pa_load(const PrefillParams& p, const int* table, int kvh, int base,
                                         int end, PaBlockRegs<D>& r) {
   using R = PaBlockRegs<D>;
@@ -82,39 +82,6 @@ __device__ __forceinline__ void pa_load(const PrefillParams& p, const int* table
   const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const __amdgpu_buffer_rsrc_t rk = buffer_resource(p.k, p.pool_bytes);
   const __amdgpu_buffer_rsrc_t rv = buffer_resource(p.v, p.pool_bytes);
-  if constexpr (OFFS) {
-    // `table` holds each page's byte offset for this kv head (kBufferAbsent
-    // for an absent page) and the page size is a power of two of at least 4:
-    // a 4-position V group lies in one page, so it costs one lookup.
-    const int shift = p.page_shift, mask = p.page_size - 1;
-    auto page_off = [&](int pos) -> unsigned {
-      return (unsigned)table[pos < end ? pos >> shift : 0];
-    };
-#pragma unroll
-    for (int i = 0; i < R::kPer; ++i) {
-      const int item = tid + i * kPaThreads;
-      const int pos = base + item / CH;
-      const unsigned off = page_off(pos);
-      const bool ok = pos < end && off != kBufferAbsent &&
-                      (R::kItems % kPaThreads == 0 || item < R::kItems);
-      r.k[i] = buffer_load_h8(
-          rk, ok ? off + (unsigned)(((pos & mask) * D + 8 * (item % CH)) * 2) : kBufferAbsent);
-    }
-#pragma unroll
-    for (int i = 0; i < R::vPer; ++i) {
-      const int item = tid + i * kPaThreads;
-      const int quad = item % (kPaBlock / 4), octet = item / (kPaBlock / 4);
-      const int pos0 = base + 4 * quad;
-      const unsigned off = page_off(pos0);
-      const unsigned row0 = off + (unsigned)(((pos0 & mask) * D + 8 * octet) * 2);
-      const bool group_ok = off != kBufferAbsent && (R::vItems % kPaThreads == 0 || item < R::vItems);
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        r.v[q][i] = buffer_load_h8(
-            rv, group_ok && pos0 + q < end ? row0 + (unsigned)(q * D * 2) : kBufferAbsent);
-    }
-    return;
-  }
   const bool pow2 = p.page_shift >= 0;
   // Element offset of (pos, 8-element column), or -1 when absent; computed
   // with selects only (table[0] exists whenever end > 0).
@@ -257,8 +224,8 @@ __device__ __forceinline__ void pa_compute(const PrefillParams& p, const half_t*
 
 // TLDS: the request's block table is staged in LDS (dynamic, max_pages
 // entries) so a block's K/V addresses need no global round trip first.
-// BUF: see pa_load.  With TLDS, BUF and a power-of-two page size of at
-// least 4 the LDS table holds byte offsets (pa_load's OFFS form).
+// BUF: see pa_load.  Serves what prefill_tile_kernel does not: pools of 4 GiB
+// and more, and block tables past kPtTable.
 template <int D, bool TLDS, bool BUF>
 __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillParams p) {
   constexpr int KS = D / 32;  // k-steps of the score product
@@ -307,7 +274,6 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
     if (p.row_table && p.row_table[token] != tile_table) len = -1;
   }
 
-  const bool offs = TLDS && BUF && p.page_shift >= 2;  // workgroup-uniform
   // Attended extent of the tile and the first absent page below it.
   if (threadIdx.x == 0) {
     s_bounds[0] = 0;
@@ -324,14 +290,7 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
     for (int i = threadIdx.x; i < pages; i += kPaThreads) {
       const int page = request_table[i];
       const bool ok = page >= 0 && page < p.pool_pages;
-      if (TLDS) {
-        if (offs)
-          s_table[i] = (int)(ok ? (unsigned)(((long)page * p.page_stride +
-                                              (long)kvh * p.head_stride) * 2)
-                                : kBufferAbsent);
-        else
-          s_table[i] = page;
-      }
+      if (TLDS) s_table[i] = page;
       if (!ok) first_bad = min(first_bad, i);
     }
     if (first_bad != 0x7fffffff) atomicMin(&s_bounds[1], first_bad);
@@ -360,10 +319,7 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
   // and land during its compute.  (Two or three blocks in flight measured
   // no faster.)
   PaBlockRegs<D> regs;
-  auto load = [&](int at) {
-    if (offs) pa_load<D, BUF, TLDS && BUF>(p, table, kvh, at, end, regs);
-    else pa_load<D, BUF, false>(p, table, kvh, at, end, regs);
-  };
+  auto load = [&](int at) { pa_load<D, BUF>(p, table, kvh, at, end, regs); };
   load(0);
   for (int base = 0; base < end; base += kPaBlock) {
     __syncthreads();  // the previous block's LDS reads are done
@@ -384,6 +340,362 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
     const h4 val = {(half_t)(o[t][0] * inv), (half_t)(o[t][1] * inv), (half_t)(o[t][2] * inv),
                     (half_t)(o[t][3] * inv)};
     *reinterpret_cast<h4*>(orow + 16 * t + 4 * g) = val;
+  }
+}
+
+// ------------------------------------------------ staged by LDS loads
+// The kernel for block tables that fit in LDS and pools below 4 GiB.  Tiles of
+// 64 query vectors as above and blocks of 32 PG positions (PG 2 or 4): each of
+// the 2 PG waves holds 32 query vectors and takes 32 of the block's positions
+// (wave = vector half + 2 * position group), so a K or V fragment read from
+// LDS feeds two score or output tiles; the 16-vector form above reads K and V
+// once per wave, twice the LDS time its MFMAs take.  K and V rows go to LDS as they lie in
+// the pages, by buffer loads with the LDS flag, one block ahead of the MFMAs
+// with one barrier per block; V^T fragments come from ds_read_b64_tr_b16 (a
+// 16-lane group's result lane n, element e is the n-th 16-bit value of the
+// 8-byte run its source lane 4e + n/4 points at), not from a transposing
+// store.  Rows are swizzled in 16-byte chunks (K) and 32-byte units (V) so
+// that operand reads spread over the banks.
+//
+// Softmax per wave over its own positions: weights 2^(s - m) with m raised
+// only when a score passes it by more than 8 (so they stay below 2^8 and the
+// outputs are seldom rescaled); their sum is one more MFMA over the rounded
+// weights.  The position groups meet in LDS at the end.
+//
+// MI355X, against the 16-vector kernel: 512 tokens at 3584 (GQA 4) 105 -> 48
+// us, 2048 tokens (MHA) 96 -> 68 (510 TFLOP/s), head dim 64, 1024 at 1024
+// 50 -> 27.  What bounds it now is the softmax's VALU work beside the MFMAs,
+// and for few blocks the latency of one block's loads.
+constexpr size_t kPtTable = 28 * 1024;  // block-table bytes beside 128 KiB of buffers
+
+// Maximum over the four lane groups of a wave (lanes l, l + 16, l + 32, l + 48),
+// by exchanging 16- and 32-lane rows of two copies.  (The exchanged words go
+// through scalars: __builtin_bit_cast of a vector element reads element 0.)
+__device__ __forceinline__ float max_over_groups(float v) {
+  const unsigned x = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const unsigned a0 = a[0], a1 = a[1];
+  v = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+  const unsigned y = __builtin_bit_cast(unsigned, v);
+  const auto b = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  const unsigned b0 = b[0], b1 = b[1];
+  return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
+
+template <int D, int PG>
+__global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(PrefillParams p) {
+  constexpr int KS = D / 32, DT = D / 16;
+  constexpr int BLOCK = 32 * PG, THREADS = 2 * PG * kWave;
+  constexpr int CH = D / 8, RPI = kWave / CH, QI = 16 / RPI;  // chunks a row, rows a load, loads
+  __shared__ __attribute__((aligned(16))) half_t s_even[2 * BLOCK * D];  // K rows, V rows
+  __shared__ __attribute__((aligned(16))) half_t s_odd[2 * BLOCK * D];
+  __shared__ int s_bounds[2];
+  extern __shared__ int s_table[];
+  typedef __attribute__((address_space(3))) void lds_void;
+
+  const int id = blockIdx.x;
+  int kvh, tile;
+  if (p.kv_heads % 8 == 0) {
+    const int xcd = id % 8, r = id / 8;
+    kvh = xcd + 8 * (r / p.tiles);
+    tile = p.tiles - 1 - r % p.tiles;
+  } else {
+    kvh = id / p.tiles;
+    tile = p.tiles - 1 - id % p.tiles;
+  }
+  const int active = min(p.active[0], p.rows);
+  const int t0 = tile * p.tokens_per_tile;
+  if (t0 >= active) return;
+  const int tile_table = p.row_table ? p.row_table[t0] : 0;
+  if (tile_table < 0 || tile_table >= p.table_rows) return;
+  const int32_t* request_table = p.table + (size_t)tile_table * p.max_pages;
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int vh = wave & 1, ph = wave >> 1;  // vector half, position group
+  const int j = lane & 15, g = lane >> 4;
+  const int capacity = p.page_size * p.max_pages;
+  int token[2], head[2], len[2];
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    const int vec = 32 * vh + 16 * v + j;
+    token[v] = t0 + vec / p.group;
+    head[v] = kvh * p.group + vec % p.group;
+    len[v] = 0;
+    if (vec < p.tokens_per_tile * p.group && token[v] < active) {
+      len[v] = p.valid[token[v]];
+      if (len[v] < 1 || len[v] > capacity) len[v] = -1;  // no output for this query
+      if (p.row_table && p.row_table[token[v]] != tile_table) len[v] = -1;
+    }
+  }
+  if (threadIdx.x == 0) {
+    s_bounds[0] = 0;
+    s_bounds[1] = 0x7fffffff;
+  }
+  __syncthreads();
+  if (g == 0 && max(len[0], len[1]) > 0) atomicMax(&s_bounds[0], max(len[0], len[1]));
+  __syncthreads();
+  const int end = s_bounds[0];
+  if (end == 0) return;
+  {
+    // the table in LDS: byte offset of each page for this kv head
+    const int pages = (end + p.page_size - 1) / p.page_size;
+    int first_bad = 0x7fffffff;
+    for (int i = threadIdx.x; i < pages; i += THREADS) {
+      const int page = request_table[i];
+      const bool ok = page >= 0 && page < p.pool_pages;
+      s_table[i] = (int)(ok ? (unsigned)(((long)page * p.page_stride + (long)kvh * p.head_stride) * 2)
+                            : kBufferAbsent);
+      if (!ok) first_bad = min(first_bad, i);
+    }
+    if (first_bad != 0x7fffffff) atomicMin(&s_bounds[1], first_bad);
+  }
+  __syncthreads();
+  const long bad_from = (long)s_bounds[1] * p.page_size;  // positions at/after: absent page
+
+  const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  h8 qb[2][KS];
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    const half_t* qrow = p.q + ((size_t)token[v] * p.q_heads + head[v]) * D;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qb[v][s] = len[v] > 0 ? load_h8(qrow + 32 * s + 8 * g) : zero;
+  }
+
+  // stage loads: load q of this wave moves rows 16 wave + RPI q ... of the
+  // block, lane l slot l % CH of row l / CH
+  const __amdgpu_buffer_rsrc_t rk = buffer_resource(p.k, p.pool_bytes);
+  const __amdgpu_buffer_rsrc_t rv = buffer_resource(p.v, p.pool_bytes);
+  const int slot = lane % CH;
+  auto load = [&](int base, half_t* buf) {
+    int page[QI], row[QI];
+    if (p.page_shift >= 0) {
+#pragma unroll
+      for (int q = 0; q < QI; ++q) {
+        const int pos = base + 16 * wave + RPI * q + lane / CH;
+        page[q] = pos >> p.page_shift;
+        row[q] = pos & (p.page_size - 1);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < QI; ++q) {
+        const int pos = base + 16 * wave + RPI * q + lane / CH;
+        page[q] = pos / p.page_size;
+        row[q] = pos - page[q] * p.page_size;
+      }
+    }
+    unsigned off[QI];
+#pragma unroll
+    for (int q = 0; q < QI; ++q) {
+      const bool in = base + 16 * wave + RPI * q + lane / CH < end;
+      const unsigned entry = (unsigned)s_table[in ? page[q] : 0];
+      off[q] = in ? entry : kBufferAbsent;
+    }
+#pragma unroll
+    for (int q = 0; q < QI; ++q) {
+      const int R = 16 * wave + RPI * q + lane / CH;
+      const bool ok = off[q] != kBufferAbsent;
+      const unsigned at = off[q] + (unsigned)(row[q] * D * 2);
+      const int kc = D == 128 ? slot ^ (R & 15) : slot ^ ((R >> 1) & 7);
+      const int vu = (slot >> 1) ^ (D == 128 ? R & 7 : (R >> 1) & 3);
+      half_t* to = buf + (16 * wave + RPI * q) * D;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rk, (lds_void*)to, 16, ok ? (int)(at + 16u * kc) : (int)kBufferAbsent, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rv, (lds_void*)(to + BLOCK * D), 16,
+          ok ? (int)(at + 32u * vu + 16u * (slot & 1)) : (int)kBufferAbsent, 0, 0, 0);
+    }
+  };
+
+  f4 o[2][DT], lsum[2];
+  float m[2];
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    m[v] = -INFINITY;
+    lsum[v] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[v][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  // Longest and shortest length of the wave's live queries: blocks past the
+  // one are skipped, blocks below the other need no mask.
+  int wave_max = max(len[0], len[1]);
+  int wave_min = min(len[0] > 0 ? len[0] : 0x7fffffff, len[1] > 0 ? len[1] : 0x7fffffff);
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    wave_max = max(wave_max, __shfl_xor(wave_max, off, kWave));
+    wave_min = min(wave_min, __shfl_xor(wave_min, off, kWave));
+  }
+  wave_max = __builtin_amdgcn_readfirstlane(wave_max);
+  wave_min = __builtin_amdgcn_readfirstlane(wave_min);
+  const h8 ones = {(half_t)1.0f, (half_t)1.0f, (half_t)1.0f, (half_t)1.0f,
+                   (half_t)1.0f, (half_t)1.0f, (half_t)1.0f, (half_t)1.0f};
+
+  // the wave's K and V^T fragments of a staged block
+  struct Frags {
+    h8 k[2][KS], v[DT];
+  };
+  auto read = [&](const half_t* buf, Frags& f) {
+    const half_t* sk = buf + 32 * ph * D;
+    const char* sv = reinterpret_cast<const char*>(buf + (BLOCK + 32 * ph) * D);
+    typedef half_t v4h __attribute__((ext_vector_type(4)));
+    typedef __fp16 v4fp16 __attribute__((__vector_size__(8)));
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int c = D == 128 ? (4 * s + g) ^ j : (4 * s + g) ^ ((j >> 1) & 7);
+        f.k[t][s] = *reinterpret_cast<const h8*>(sk + (16 * t + j) * D + 8 * c);
+      }
+    // k slot 8g + e is position 4g + e (e < 4) or 16 + 4g + (e - 4) of the 32
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      v4h part[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int R = 16 * h + 4 * g + (j >> 2);
+        const int unit = t ^ (D == 128 ? R & 7 : (R >> 1) & 3);
+        part[h] = __builtin_bit_cast(
+            v4h, __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+                     reinterpret_cast<__attribute__((address_space(3))) v4fp16*>(
+                         (__attribute__((address_space(3))) char*)sv + R * D * 2 + 32 * unit +
+                         8 * (j & 3))));
+      }
+      f.v[t] = __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  };
+  auto compute = [&](int base, const Frags& f) {
+    const int first = base + 32 * ph;  // this wave's 32 positions
+    f4 sc[2][2];                       // [vector tile][position tile]
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        sc[v][t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          sc[v][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.k[t][s], qb[v][s], sc[v][t], 0, 0, 0);
+      }
+    if (first + 32 > wave_min) {  // wave-uniform
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (first + 16 * t + 4 * g + r >= len[v]) sc[v][t][r] = -INFINITY;
+    }
+    float next[2];
+    bool raise = false;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      float b = fmaxf(fmaxf(fmaxf(sc[v][0][0], sc[v][0][1]), fmaxf(sc[v][0][2], sc[v][0][3])),
+                      fmaxf(fmaxf(sc[v][1][0], sc[v][1][1]), fmaxf(sc[v][1][2], sc[v][1][3])));
+      b = max_over_groups(b) * p.scale_log2;
+      // the first finite score, or one that passes m by more than 2^8
+      const bool up = b > m[v] + 8.0f;
+      next[v] = up ? b : m[v];
+      raise = raise || up;
+    }
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        const float alpha = next[v] == m[v] ? 1.0f : fast_exp2(m[v] - next[v]);
+        m[v] = next[v];
+        lsum[v] *= alpha;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[v][t] *= alpha;
+      }
+    }
+    h8 pb[2];
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const float shift = m[v] == -INFINITY ? 0.0f : m[v];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          pb[v][4 * t + r] = (half_t)fast_exp2(__fmaf_rn(sc[v][t][r], p.scale_log2, -shift));
+      lsum[v] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb[v], lsum[v], 0, 0, 0);
+    }
+    // O^T[d][query] += V^T[d][pos] P^T[pos][query]
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int v = 0; v < 2; ++v)
+        o[v][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.v[t], pb[v], o[v][t], 0, 0, 0);
+  };
+
+  // One block out of `now`, the next one's loads into `then`.  The fragments
+  // are read before those loads go out (the compiler has a transposing read
+  // wait for every LDS load in flight), and from two named buffers (with one
+  // array and an index it would have every LDS read wait for them).
+  auto step = [&](int base, const half_t* now, half_t* then) {
+    // this wave's loads of the block have landed, and every wave is done
+    // reading the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    Frags f;
+    read(now, f);
+    if (base + BLOCK < end) load(base + BLOCK, then);
+    if (base + 32 * ph < wave_max) compute(base, f);
+  };
+  load(0, s_even);
+  for (int base = 0; base < end; base += 2 * BLOCK) {
+    step(base, s_even, s_odd);
+    if (base + BLOCK < end) step(base + BLOCK, s_odd, s_even);
+  }
+
+  // the position groups meet: the others hand group 0 their sums through LDS
+  __syncthreads();
+  constexpr int kHand = (2 + 4 * DT) * kWave;  // floats a vector tile hands over
+  static_assert((PG - 1) * 2 * kHand * 4 <= 2 * BLOCK * D * 2, "the handed sums fit one buffer");
+  float* hand = reinterpret_cast<float*>(vh ? s_odd : s_even) + lane;
+  if (ph > 0) {
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      float* at = hand + (2 * (ph - 1) + v) * kHand;
+      at[0] = m[v];
+      at[kWave] = lsum[v][0];
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) at[(2 + 4 * t + r) * kWave] = o[v][t][r];
+    }
+  }
+  __syncthreads();
+  if (ph > 0) return;
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    if (len[v] <= 0 || len[v] > bad_from) continue;
+    float top = m[v];
+#pragma unroll
+    for (int q = 0; q < PG - 1; ++q) top = fmaxf(top, hand[(2 * q + v) * kHand]);
+    // a group without positions of this query holds -inf and zeros
+    const float own = m[v] == -INFINITY ? 0.0f : fast_exp2(m[v] - top);
+    float sum = own * lsum[v][0];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[v][t] *= own;
+#pragma unroll
+    for (int q = 0; q < PG - 1; ++q) {
+      const float* at = hand + (2 * q + v) * kHand;
+      const float other = at[0];
+      const float scale = other == -INFINITY ? 0.0f : fast_exp2(other - top);
+      sum += scale * at[kWave];
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[v][t][r] += scale * at[(2 + 4 * t + r) * kWave];
+    }
+    const float inv = 1.0f / sum;
+    half_t* orow = p.out + ((size_t)token[v] * p.q_heads + head[v]) * D;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      const h4 val = {(half_t)(o[v][t][0] * inv), (half_t)(o[v][t][1] * inv),
+                      (half_t)(o[v][t][2] * inv), (half_t)(o[v][t][3] * inv)};
+      *reinterpret_cast<h4*>(orow + 16 * t + 4 * g) = val;
+    }
   }
 }
 
@@ -451,25 +763,42 @@ extern "C" int tmc_prefill_attention_rows_f16(const void* q, const void* key_poo
                             (size_t)head_dim * (kPaBlock + kVPad) * 2 + 16;
   const size_t table_lds = (size_t)max_pages * 4;
   const bool tlds = static_lds + table_lds <= kPaMaxLds;
-  const size_t dyn = tlds ? table_lds : 0;
+  const bool buf = (uint64_t)pool_pages * (uint64_t)page_stride * 2 < kBufferAbsent;
+  const size_t dyn = tlds && !buf ? table_lds : 0;
   const hipStream_t s = as_stream(stream);
   const uint64_t pool_bytes = (uint64_t)pool_pages * (uint64_t)page_stride * 2;
-  const bool buf = pool_bytes < kBufferAbsent;
   p.pool_bytes = buf ? (unsigned)pool_bytes : 0u;
+  // 16-byte loads into LDS need 16-byte rows
+  const bool rows16 = aligned16(key_pool) && aligned16(value_pool) && page_stride % 8 == 0 &&
+                      head_stride % 8 == 0;
+  if (buf && rows16 && table_lds <= kPtTable) {
+    // Four position groups (8 waves, 128 positions a block) where a launch has
+    // at most one block per CU and contexts may be long: 512 tokens at 3584,
+    // GQA 4: 48 us against 63 with two groups, 16 at 3000 37 against 49; with
+    // more blocks than CUs two 4-wave blocks share a CU and two groups win
+    // (2048 tokens MHA 68 against 75), and below about 500 positions the
+    // longer hand-over costs more than it saves (200 tokens 8.8 against 10.2).
+    const bool four = grid.x <= 256 && page_size * max_pages > 1024;
+#define TMC_PT_LAUNCH(DIM, PG) \
+  hipLaunchKernelGGL((prefill_tile_kernel<DIM, PG>), grid, dim3(2 * PG * kWave), table_lds, s, p)
+    if (head_dim == 128) {
+      if (four) TMC_PT_LAUNCH(128, 4); else TMC_PT_LAUNCH(128, 2);
+    } else {
+      if (four) TMC_PT_LAUNCH(64, 4); else TMC_PT_LAUNCH(64, 2);
+    }
+#undef TMC_PT_LAUNCH
+    return check_launch("prefill_tile_kernel");
+  }
 #define TMC_PA_LAUNCH(DIM, T, B)                                                                  \
   hipLaunchKernelGGL((prefill_attention_kernel<DIM, T, B>), grid, dim3(kPaThreads), dyn, s, p)
   if (head_dim == 128) {
-    if (tlds) {
-      if (buf) TMC_PA_LAUNCH(128, true, true); else TMC_PA_LAUNCH(128, true, false);
-    } else {
-      if (buf) TMC_PA_LAUNCH(128, false, true); else TMC_PA_LAUNCH(128, false, false);
-    }
+    if (buf) TMC_PA_LAUNCH(128, false, true);
+    else if (tlds) TMC_PA_LAUNCH(128, true, false);
+    else TMC_PA_LAUNCH(128, false, false);
   } else {
-    if (tlds) {
-      if (buf) TMC_PA_LAUNCH(64, true, true); else TMC_PA_LAUNCH(64, true, false);
-    } else {
-      if (buf) TMC_PA_LAUNCH(64, false, true); else TMC_PA_LAUNCH(64, false, false);
-    }
+    if (buf) TMC_PA_LAUNCH(64, false, true);
+    else if (tlds) TMC_PA_LAUNCH(64, true, false);
+    else TMC_PA_LAUNCH(64, false, false);
   }
 #undef TMC_PA_LAUNCH
   return check_launch("prefill_attention_kernel");
