@@ -18,8 +18,9 @@
 // of which writes back and invalidates the XCD's L2, measured several times
 // slower.)
 //
-// D = 128 runs attn_mfma_kernel (scores from v_mfma_f32_16x16x32_f16, see the
-// comment above it); smaller heads run attn_partial_kernel: RL = D/8 lanes
+// D = 128, and D = 64 where launch_plan says so, runs attn_mfma_kernel (scores
+// from v_mfma_f32_16x16x32_f16, see the comment above it); the rest runs
+// attn_partial_kernel: RL = D/8 lanes
 // hold one position's 16-byte slices, so one 16-byte load covers NR = 64/RL
 // consecutive positions, a wave tile is J = 4 such loads, and rows are
 // folded together once per split (cross-row shuffles).
@@ -65,8 +66,8 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kTilesPerWave = 2;  // VALU kernel (D < 128)
-// D == 128 kernel: a wave step is kMfmaTiles 16-position MFMA tiles whose
+constexpr int kTilesPerWave = 2;  // VALU kernel
+// MFMA kernel: a wave step is kMfmaTiles 16-position MFMA tiles whose
 // K/V loads are all issued before the first MFMA.  (Keeping a second step's
 // loads in flight was measured slower: the extra registers halve occupancy.)
 // Positions per split are chosen per launch from 128 ... 1024 (chunk_for).
@@ -104,7 +105,8 @@ struct AttnParams {
   int page_shift;         // log2(page_size) when it is a power of two, else -1
   long pool_pages;        // paged: pages in each pool (0 = unknown, no bound check)
   int chunk;              // positions per split
-  int waves;              // waves per block (D = 128: kWaves, or kWideWaves for one split)
+  int waves;              // waves per block (kWaves, or kMidWaves / kWideWaves for one split)
+  bool valu;              // attn_partial_kernel (always below D = 64)
   unsigned kv_bytes;      // bytes of the K (and of the V) buffer when < 4 GiB, else 0
   float scale_log2;       // (1/sqrt(D)) * log2(e)
   int* arrivals;          // D = 128 multi-split: [batch][kv_heads] split counters (workspace start)
@@ -211,7 +213,7 @@ __device__ int dealt_unit(const AttnParams& p, int slot, int rows, int splits, i
 // lengths differ, keep the capacity's chunk.
 template <bool PAGED>
 __device__ __forceinline__ int mfma_chunk(const AttnParams& p, int valid) {
-  if (PAGED || p.max_splits <= 1) return p.chunk;
+  if (PAGED || p.max_splits <= 1 || p.valu) return p.chunk;
   const int steps = (valid + kMfmaStep - 1) / kMfmaStep;
   return (steps + p.max_splits - 1) / p.max_splits * kMfmaStep;
 }
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
   fetch(0);
   const int valid = valid_length<PAGED>(p, b);
   if (valid < 1 || valid > p.capacity) return;
-  const int chunk = D == 128 ? mfma_chunk<PAGED>(p, valid) : p.chunk;
+  const int chunk = D >= 64 ? mfma_chunk<PAGED>(p, valid) : p.chunk;
   const int nsplit = (valid + chunk - 1) / chunk;
   if (nsplit <= 1) return;
   float mx = -INFINITY, lsum = 0.0f, osum = 0.0f;
@@ -484,8 +486,9 @@ __global__ __launch_bounds__(kThreads) void attn_partial_kernel(AttnParams p) {
   finish_split<D, GROUP, PAGED>(p, b, kvh, split, nsplit, bad, s_m, s_l, s_o);
 }
 
-// ---------------------------------------------------------------- D = 128
-// Split partial for D = 128: grid (split, kv head, request).  Wave w takes
+// ------------------------------------------------------- D = 128 and D = 64
+// Split partial on MFMA (written for D = 128; D = 64 halves the k-steps, the
+// loads of a tile and the 16-dim output tiles): grid (split, kv head, request).  Wave w takes
 // the steps w, w + 4, ... of its split; a step is kMfmaTiles tiles of 16
 // positions.
 //
@@ -521,9 +524,26 @@ __device__ __forceinline__ h8 buffer_h8(__amdgpu_buffer_rsrc_t r, unsigned byte_
                                                                       NT ? 2 : 0));
 }
 
-template <int MODE>
+// Whole-row loads: one instruction reads RP rows of D halves, lane (j, g) the
+// 16-byte chunk lane_chunk of row lane_row (D = 128: 4 rows of 16 chunks; D =
+// 64: 8 rows of 8).
+template <int D> constexpr int rows_per_load() { return 512 / D; }
+template <int D> __device__ __forceinline__ int lane_row(int j, int g) {
+  return D == 128 ? g : 2 * g + (j >> 3);
+}
+template <int D> __device__ __forceinline__ int lane_chunk(int j) { return D == 128 ? j : j & 7; }
+// LDS slots of a row's 16-byte chunks (K) and 32-byte units (V): 16 rows'
+// reads of one chunk, and a transposing read's rows, fall on distinct banks.
+template <int D> __device__ __forceinline__ int chunk_swizzle(int row) {
+  return D == 128 ? row & 15 : (row >> 1) & 7;
+}
+template <int D> __device__ __forceinline__ int unit_swizzle(int row) {
+  return D == 128 ? row & 7 : (row >> 1) & 3;
+}
+
+template <int D, int MODE>
 struct KvStep {
-  h8 k[kMfmaTiles][4], v[kMfmaTiles][4];
+  h8 k[kMfmaTiles][D / 32], v[kMfmaTiles][D / 32];
   long tile[kMfmaTiles];  // element offset of each tile's first position, -1 = absent
 };
 
@@ -533,20 +553,23 @@ __device__ __forceinline__ bool page_ok(const AttnParams& p, int page) {
 }
 
 // Element offset of position `pos` (MODE 2 lookup), -1 when absent.
+template <int D>
 __device__ __forceinline__ long paged_offset(const AttnParams& p, const int* s_pages, int page0,
                                              int kvh, int pos, int end) {
   if (pos >= end) return -1;
   const int page = s_pages[page_of(p, pos) - page0];
   if (!page_ok<2>(p, page)) return -1;
   return (long)page * p.page_stride + (long)kvh * p.head_stride +
-         (long)slot_in_page(p, pos) * 128;
+         (long)slot_in_page(p, pos) * D;
 }
 
-template <int MODE, bool VIA = false>
+template <int D, int MODE, bool VIA = false>
 __device__ __forceinline__ void issue_step(const AttnParams& p, const int* s_pages, int page0,
                                            size_t cbase, int kvh, int p0, int end, int j, int g,
                                            __amdgpu_buffer_rsrc_t rk, __amdgpu_buffer_rsrc_t rv,
-                                           KvStep<MODE>& st) {
+                                           KvStep<D, MODE>& st) {
+  constexpr int RP = rows_per_load<D>(), QL = D / 32;
+  const int lr = lane_row<D>(j, g), lc = lane_chunk<D>(j);
   const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t) {
@@ -555,7 +578,7 @@ __device__ __forceinline__ void issue_step(const AttnParams& p, const int* s_pag
       long tile = -1;
       if (tp < end) {
         if constexpr (MODE == 0) {
-          tile = (long)(cbase + (size_t)tp * 128);
+          tile = (long)(cbase + (size_t)tp * D);
         } else {
           // The tile's page id is the same for every lane: in a scalar
           // register the branch on it stays scalar, so the loads below are
@@ -564,7 +587,7 @@ __device__ __forceinline__ void issue_step(const AttnParams& p, const int* s_pag
           const int page = __builtin_amdgcn_readfirstlane(s_pages[page_of(p, tp) - page0]);
           if (page_ok<1>(p, page))
             tile = (long)page * p.page_stride + (long)kvh * p.head_stride +
-                   (long)slot_in_page(p, tp) * 128;
+                   (long)slot_in_page(p, tp) * D;
         }
       }
       st.tile[t] = tile;
@@ -574,77 +597,83 @@ __device__ __forceinline__ void issue_step(const AttnParams& p, const int* s_pag
       const unsigned tb = tile < 0 ? 0u : (unsigned)(tile * 2);
       const unsigned tmask = tile < 0 ? kAbsent : 0u;
       if constexpr (VIA) {
-        // whole rows: load q reads positions 4q .. 4q + 3 of the tile, lane
-        // (j, g) the 16-byte chunk j of position 4q + g (8 full cache lines
-        // per load); consume_step re-lays them in the MFMA operand order
+        // whole rows: load q reads positions RP q ... of the tile (8 full
+        // cache lines per load); consume_step re-lays them in the MFMA
+        // operand order
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const unsigned rmask = tmask | (tp + 4 * q + g < end ? 0u : kAbsent);
-          st.k[t][q] = buffer_h8<MODE == 0>(rk, (tb + (unsigned)(4 * q + g) * 256u + 16u * j) | rmask);
+        for (int q = 0; q < QL; ++q) {
+          const unsigned rmask = tmask | (tp + RP * q + lr < end ? 0u : kAbsent);
+          st.k[t][q] =
+              buffer_h8<MODE == 0>(rk, (tb + (unsigned)(RP * q + lr) * (2u * D) + 16u * lc) | rmask);
         }
       } else {
         const unsigned kmask = tmask | (tp + j < end ? 0u : kAbsent);
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-          st.k[t][s] = buffer_h8<MODE == 0>(rk, (tb + (unsigned)j * 256u + 16u * (4 * s + g)) | kmask);
+        for (int s = 0; s < QL; ++s)
+          st.k[t][s] =
+              buffer_h8<MODE == 0>(rk, (tb + (unsigned)j * (2u * D) + 16u * (4 * s + g)) | kmask);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const unsigned vmask = tmask | (tp + 4 * i + g < end ? 0u : kAbsent);
-        st.v[t][i] = buffer_h8<MODE == 0>(rv, (tb + (unsigned)(4 * i + g) * 256u + 16u * j) | vmask);
+      for (int i = 0; i < QL; ++i) {
+        const unsigned vmask = tmask | (tp + RP * i + lr < end ? 0u : kAbsent);
+        st.v[t][i] =
+            buffer_h8<MODE == 0>(rv, (tb + (unsigned)(RP * i + lr) * (2u * D) + 16u * lc) | vmask);
       }
     } else {
       st.tile[t] = tp < end ? 0 : -1;
-      const long krow = paged_offset(p, s_pages, page0, kvh, tp + j, end);
+      const long krow = paged_offset<D>(p, s_pages, page0, kvh, tp + j, end);
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int s = 0; s < QL; ++s)
         st.k[t][s] = krow >= 0 ? load_h8(p.k + krow + 8 * (4 * s + g)) : zero;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const long vrow = paged_offset(p, s_pages, page0, kvh, tp + 4 * i + g, end);
-        st.v[t][i] = vrow >= 0 ? load_h8(p.v + vrow + 8 * j) : zero;
+      for (int i = 0; i < QL; ++i) {
+        const long vrow = paged_offset<D>(p, s_pages, page0, kvh, tp + RP * i + lr, end);
+        st.v[t][i] = vrow >= 0 ? load_h8(p.v + vrow + 8 * lc) : zero;
       }
     }
   }
 }
 
-template <int GROUP, int MODE, bool VIA = false>
+template <int D, int GROUP, int MODE, bool VIA = false>
 __device__ __forceinline__ void consume_step(const AttnParams& p, const int* s_pages, int page0,
-                                             const KvStep<MODE>& st, const h8 (&qb)[4], int p0,
-                                             int end, int j, int g, float (*s_pw)[GROUP],
+                                             const KvStep<D, MODE>& st, const h8 (&qb)[D / 32],
+                                             int p0, int end, int j, int g, float (*s_pw)[GROUP],
                                              float& m, float& lsum, float (&o)[GROUP][8],
                                              h8* s_k = nullptr) {
+  constexpr int RP = rows_per_load<D>(), QL = D / 32, CH = D / 8;
+  const int lr = lane_row<D>(j, g);
   float sc[kMfmaTiles][4];
   float tile_max = -INFINITY;
-  h8 kf[kMfmaTiles][4];
+  h8 kf[kMfmaTiles][QL];
   if constexpr (VIA) {
-    // this wave's LDS slice, 16 rows x 16 chunks per tile; chunk c of row r
-    // at slot c ^ r, so the row-wise stores and the column-wise operand
-    // reads both touch 16 distinct bank groups per 16 lanes
+    // this wave's LDS slice, 16 rows x CH chunks per tile, swizzled so that
+    // the row-wise stores and the column-wise operand reads both touch 16
+    // distinct bank groups per 16 lanes
 #pragma unroll
     for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = 4 * q + g;
-        s_k[t * 256 + r * 16 + (j ^ r)] = st.k[t][q];
+      for (int q = 0; q < QL; ++q) {
+        const int r = RP * q + lr;
+        s_k[(t * 16 + r) * CH + (lane_chunk<D>(j) ^ chunk_swizzle<D>(r))] = st.k[t][q];
       }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[t][s] = s_k[t * 256 + j * 16 + ((4 * s + g) ^ j)];
+      for (int s = 0; s < QL; ++s)
+        kf[t][s] = s_k[(t * 16 + j) * CH + ((4 * s + g) ^ chunk_swizzle<D>(j))];
     __builtin_amdgcn_wave_barrier();
   } else {
 #pragma unroll
     for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) kf[t][s] = st.k[t][s];
+      for (int s = 0; s < QL; ++s) kf[t][s] = st.k[t][s];
   }
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t) {
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < QL; ++s)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[t][s], qb[s], acc, 0, 0, 0);
     const int tp = p0 + 16 * t;
 #pragma unroll
@@ -681,10 +710,10 @@ __device__ __forceinline__ void consume_step(const AttnParams& p, const int* s_p
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < QL; ++i) {
       float pv[GROUP];
 #pragma unroll
-      for (int h = 0; h < GROUP; ++h) pv[h] = s_pw[16 * t + 4 * i + g][h];
+      for (int h = 0; h < GROUP; ++h) pv[h] = s_pw[16 * t + RP * i + lr][h];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float v = (float)st.v[t][i][e];
@@ -707,44 +736,48 @@ __device__ __forceinline__ void consume_step(const AttnParams& p, const int* s_p
 // just as the score MFMA left them: lane (head j, group g) holds positions
 // 4g .. 4g+3 of both 16-position tiles, the same k order.  oacc[db][r] is
 // O[head 4g + r][16 db + j], summed over the positions of the steps so far.
-template <int GROUP, int MODE>
-__device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvStep<MODE>& st,
-                                                 const h8 (&qb)[4], int p0, int end, int j, int g,
-                                                 float& m, float& lsum, f4 (&oacc)[8], h8* s_k) {
+template <int D, int GROUP, int MODE>
+__device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvStep<D, MODE>& st,
+                                                 const h8 (&qb)[D / 32], int p0, int end, int j,
+                                                 int g, float& m, float& lsum,
+                                                 f4 (&oacc)[D / 16], h8* s_k) {
+  constexpr int RP = rows_per_load<D>(), QL = D / 32, CH = D / 8;
+  const int lr = lane_row<D>(j, g), lc = lane_chunk<D>(j);
   static_assert(MODE != 2 && GROUP <= 16, "whole-row K/V forms, at most 16 heads per kv head");
   typedef half_t v4h __attribute__((ext_vector_type(4)));
   typedef __fp16 v4fp16 __attribute__((__vector_size__(8)));
   float sc[kMfmaTiles][4];
   float tile_max = -INFINITY;
-  h8 kf[kMfmaTiles][4];
+  h8 kf[kMfmaTiles][QL];
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = 4 * q + g;
-      s_k[t * 256 + r * 16 + (j ^ r)] = st.k[t][q];
+    for (int q = 0; q < QL; ++q) {
+      const int r = RP * q + lr;
+      s_k[(t * 16 + r) * CH + (lc ^ chunk_swizzle<D>(r))] = st.k[t][q];
     }
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-    for (int s = 0; s < 4; ++s) kf[t][s] = s_k[t * 256 + j * 16 + ((4 * s + g) ^ j)];
+    for (int s = 0; s < QL; ++s)
+      kf[t][s] = s_k[(t * 16 + j) * CH + ((4 * s + g) ^ chunk_swizzle<D>(j))];
   __builtin_amdgcn_wave_barrier();
-  // V row R = 16t + 4i + g, 16-byte chunk j: unit j/2 at slot (j/2) ^ (R & 7)
+  // V row R = 16t + RP i + lr, 16-byte chunk lc: its 32-byte unit swizzled by R
   char* vb = reinterpret_cast<char*>(s_k);
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int R = 16 * t + 4 * i + g;
-      *reinterpret_cast<h8*>(vb + R * 256 + (((j >> 1) ^ (R & 7)) << 5) + ((j & 1) << 4)) =
-          st.v[t][i];
+    for (int i = 0; i < QL; ++i) {
+      const int R = 16 * t + RP * i + lr;
+      *reinterpret_cast<h8*>(vb + R * 2 * D + (((lc >> 1) ^ unit_swizzle<D>(R)) << 5) +
+                             ((lc & 1) << 4)) = st.v[t][i];
     }
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t) {
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < QL; ++s)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[t][s], qb[s], acc, 0, 0, 0);
     const int tp = p0 + 16 * t;
 #pragma unroll
@@ -759,14 +792,19 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
   const float next = fmaxf(m, tile_max);
   const float alpha = next == -INFINITY ? 1.0f : fast_exp2(m - next);
   float psum = 0.0f;
-  h8 pa;
+  // D = 64: fp16 weights and what their rounding left, so that the product
+  // keeps the fp32 weights of the VALU form (21 bits of them)
+  constexpr bool kSplitP = D != 128;
+  h8 pa, pl;
 #pragma unroll
   for (int t = 0; t < kMfmaTiles; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float pr = sc[t][r] == -INFINITY ? 0.0f : fast_exp2(sc[t][r] - next);
       psum += pr;
-      pa[4 * t + r] = (half_t)(j < GROUP ? pr : 0.0f);
+      const float pw = j < GROUP ? pr : 0.0f;
+      pa[4 * t + r] = (half_t)pw;
+      if constexpr (kSplitP) pl[4 * t + r] = (half_t)(pw - (float)pa[4 * t + r]);
     }
   lsum = lsum * alpha + psum;
   m = next;
@@ -775,23 +813,26 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
   for (int r = 0; r < 4; ++r) {
     const float ar = __shfl(alpha, 4 * g + r, kWave);
 #pragma unroll
-    for (int db = 0; db < 8; ++db) oacc[db][r] *= ar;
+    for (int db = 0; db < D / 16; ++db) oacc[db][r] *= ar;
   }
   __builtin_amdgcn_wave_barrier();
   const int s16 = j;  // source lane within the 16-lane group
 #pragma unroll
-  for (int db = 0; db < 8; ++db) {
+  for (int db = 0; db < D / 16; ++db) {
     v4h half_b[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int R = 16 * h + 4 * g + (s16 >> 2);
       half_b[h] = __builtin_bit_cast(v4h, __builtin_amdgcn_ds_read_tr16_b64_v4f16(
           reinterpret_cast<__attribute__((address_space(3))) v4fp16*>(
-              (__attribute__((address_space(3))) char*)vb + R * 256 + ((db ^ (R & 7)) << 5) +
+              (__attribute__((address_space(3))) char*)vb + R * 2 * D +
+              ((db ^ unit_swizzle<D>(R)) << 5) +
               ((s16 & 3) << 3))));
     }
     const h8 bv = __builtin_shufflevector(half_b[0], half_b[1], 0, 1, 2, 3, 4, 5, 6, 7);
     oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, bv, oacc[db], 0, 0, 0);
+    if constexpr (kSplitP)
+      oacc[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, bv, oacc[db], 0, 0, 0);
   }
   __builtin_amdgcn_wave_barrier();
 }
@@ -809,9 +850,8 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
 // marked slot leaves the output untouched) and resets the counter.  No
 // block waits for another and no cache writeback or invalidate is needed:
 // every shared word is written and read with agent-scope operations.
-template <int GROUP, bool PAGED, int WAVES>
+template <int D, int GROUP, bool PAGED, int WAVES>
 __device__ void merge_if_last(const AttnParams& p, int b, int kvh, int nsplit) {
-  constexpr int D = 128;
   __shared__ int s_last;
   int* counter = p.arrivals + (size_t)b * p.kv_heads + kvh;
   __builtin_amdgcn_s_waitcnt(0);  // this thread's slot stores have completed
@@ -886,9 +926,8 @@ __device__ void merge_if_last(const AttnParams& p, int b, int kvh, int nsplit) {
   }
 }
 
-template <int GROUP, int MODE, int WAVES>
+template <int D, int GROUP, int MODE, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) {
-  constexpr int D = 128;
   constexpr bool PAGED = MODE != 0;
   __shared__ float s_m[WAVES][GROUP];
   __shared__ float s_l[WAVES][GROUP];
@@ -913,10 +952,10 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
   // 15.2-15.4 us as the direct loads with two steps in flight, which this
   // replaces.  MODE 2 looks up every position and keeps the direct loads.
   constexpr bool kVia = MODE != 2;
-  __shared__ h8 s_k[kVia ? WAVES : 1][kVia ? kMfmaTiles * 256 : 1];
+  __shared__ h8 s_k[kVia ? WAVES : 1][kVia ? kMfmaTiles * 2 * D : 1];
 
   const int kvh = blockIdx.x;
-  constexpr bool TL = TMC_ATTN_TIMELINE && MODE != 2 && (WAVES == kWaves || WAVES == kMidWaves);
+  constexpr bool TL = TMC_ATTN_TIMELINE && D == 128 && MODE != 2 && (WAVES == kWaves || WAVES == kMidWaves);
   if constexpr (TL) {
     timeline_put<TL>(0, __builtin_amdgcn_s_memrealtime());
     timeline_put<TL>(3, shader_clock());
@@ -948,11 +987,11 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
   const int j = lane & 15;
   const int g = lane >> 4;
   const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  h8 qb[4];
+  h8 qb[D / 32];
   {
     const half_t* qrow = p.q + ((size_t)b * p.q_heads + kvh * GROUP + (j < GROUP ? j : 0)) * D;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) qb[s] = j < GROUP ? load_h8(qrow + 8 * (4 * s + g)) : zero;
+    for (int s = 0; s < D / 32; ++s) qb[s] = j < GROUP ? load_h8(qrow + 8 * (4 * s + g)) : zero;
   }
   if (b >= active_rows) return;
   if (valid < 1 || valid > p.capacity) return;
@@ -984,15 +1023,15 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
   }
   float m = -INFINITY, lsum = 0.0f;
   // kPvm: oacc[db][r] = O[head 4g + r][16 db + j]; else o[h][e] = this lane's
-  // share of O[head h][8 j + e]
+  // share of O[head h][8 lane_chunk + e]
   float o[kPvm ? 1 : GROUP][8];
-  f4 oacc[kPvm ? 8 : 1];
+  f4 oacc[kPvm ? D / 16 : 1];
 #pragma unroll
   for (int h = 0; h < (kPvm ? 1 : GROUP); ++h)
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[h][e] = 0.0f;
 #pragma unroll
-  for (int db = 0; db < (kPvm ? 8 : 1); ++db) oacc[db] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int db = 0; db < (kPvm ? D / 16 : 1); ++db) oacc[db] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   const size_t cbase = ((size_t)b * p.kv_heads + kvh) * (size_t)p.capacity * D;
   const __amdgpu_buffer_rsrc_t rk = buffer_of(p.k, p.kv_bytes);
   const __amdgpu_buffer_rsrc_t rv = buffer_of(p.v, p.kv_bytes);
@@ -1002,17 +1041,17 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
   int steps = 0;
   if constexpr (TL) timeline_put<TL>(4, shader_clock());
   for (int p0 = begin + kMfmaStep * wave; p0 < end; p0 += kStride) {
-    KvStep<MODE> st;
+    KvStep<D, MODE> st;
     if constexpr (TL) if (steps < 12) timeline_put<TL>(10 + 3 * steps, shader_clock());
-    issue_step<MODE, kVia>(p, s_pages, page0, cbase, kvh, p0, end, j, g, rk, rv, st);
+    issue_step<D, MODE, kVia>(p, s_pages, page0, cbase, kvh, p0, end, j, g, rk, rv, st);
     if constexpr (TL) {
       __builtin_amdgcn_s_waitcnt(0);
       if (steps < 12) timeline_put<TL>(11 + 3 * steps, shader_clock());
     }
     if constexpr (kPvm)
-      consume_step_pvm<GROUP, MODE>(p, st, qb, p0, end, j, g, m, lsum, oacc, s_k[wave]);
+      consume_step_pvm<D, GROUP, MODE>(p, st, qb, p0, end, j, g, m, lsum, oacc, s_k[wave]);
     else
-      consume_step<GROUP, MODE, kVia>(p, s_pages, page0, st, qb, p0, end, j, g, s_pw, m, lsum, o,
+      consume_step<D, GROUP, MODE, kVia>(p, s_pages, page0, st, qb, p0, end, j, g, s_pw, m, lsum, o,
                                       s_k[kVia ? wave : 0]);
     if constexpr (TL) if (steps < 12) timeline_put<TL>(12 + 3 * steps, shader_clock());
     ++steps;
@@ -1028,17 +1067,17 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
     for (int r = 0; r < 4; ++r)
       if (4 * g + r < GROUP)
 #pragma unroll
-        for (int db = 0; db < 8; ++db) s_o[wave][4 * g + r][16 * db + j] = oacc[db][r];
+        for (int db = 0; db < D / 16; ++db) s_o[wave][4 * g + r][16 * db + j] = oacc[db][r];
   } else {
 #pragma unroll
     for (int h = 0; h < GROUP; ++h)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[h][e] = cross_sum<16>(o[h][e]);
-    if (g == 0)
+      for (int e = 0; e < 8; ++e) o[h][e] = cross_sum<D / 8>(o[h][e]);
+    if (lane_row<D>(j, g) == 0)
 #pragma unroll
       for (int h = 0; h < GROUP; ++h)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s_o[wave][h][8 * j + e] = o[h][e];
+        for (int e = 0; e < 8; ++e) s_o[wave][h][8 * lane_chunk<D>(j) + e] = o[h][e];
   }
   if (g == 0 && j < GROUP) {
     s_m[wave][j] = m;
@@ -1047,7 +1086,7 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
   __syncthreads();
   finish_split<D, GROUP, PAGED, WAVES>(p, b, kvh, split, nsplit, bad, s_m, s_l, s_o);
   if constexpr (TL) timeline_put<TL>(6, shader_clock());
-  if (nsplit > 1 && p.arrivals) merge_if_last<GROUP, PAGED, WAVES>(p, b, kvh, nsplit);
+  if (nsplit > 1 && p.arrivals) merge_if_last<D, GROUP, PAGED, WAVES>(p, b, kvh, nsplit);
   if constexpr (TL) {
     timeline_put<TL>(7, shader_clock());
     timeline_put<TL>(1, __builtin_amdgcn_s_memrealtime());
@@ -1062,46 +1101,50 @@ int launch_group(const AttnParams& params, int batch, hipStream_t stream) {
 #endif
   if (D != 128 || GROUP > 4) p.arrivals = nullptr;  // merge launch (see merge_if_last)
   const dim3 grid((unsigned)p.kv_heads, (unsigned)p.max_splits, (unsigned)batch);
-  if constexpr (D == 128) {
+#define TMC_ATTN(MODE, WAVES)                                                                    \
+  hipLaunchKernelGGL((attn_mfma_kernel<D, GROUP, MODE, WAVES>), grid, dim3(WAVES * kWave), 0,    \
+                     stream, p)
+  if constexpr (D == 64) {
+    // split_plan: whole-row forms only, wide blocks of groups up to 2 and
+    // 4-wave blocks of wider ones
+    if (p.valu) {
+      hipLaunchKernelGGL((attn_partial_kernel<D, GROUP, PAGED>), grid, dim3(kThreads), 0, stream, p);
+    } else if constexpr (GROUP <= kWideMaxGroup) {
+      TMC_ATTN(PAGED ? 1 : 0, kWideWaves);
+    } else {
+      TMC_ATTN(PAGED ? 1 : 0, kWaves);
+    }
+  } else if constexpr (D == 128) {
+    const int mode = p.kv_bytes != 0 && !PAGED ? 0 : p.kv_bytes != 0 && p.page_size % 16 == 0 ? 1 : 2;
+    if (mode == 2 && !PAGED)
+      return fail("Attention: contiguous caches of 4 GiB or more are not supported.");
     if (p.waves == kWideWaves) {
       if constexpr (GROUP <= kWideMaxGroup) {
-        const dim3 block(kWideWaves * kWave);
-        if (p.kv_bytes != 0 && !PAGED)
-          hipLaunchKernelGGL((attn_mfma_kernel<GROUP, 0, kWideWaves>), grid, block, 0, stream, p);
-        else if (p.kv_bytes != 0 && p.page_size % 16 == 0)
-          hipLaunchKernelGGL((attn_mfma_kernel<GROUP, 1, kWideWaves>), grid, block, 0, stream, p);
-        else if (PAGED)
-          hipLaunchKernelGGL((attn_mfma_kernel<GROUP, 2, kWideWaves>), grid, block, 0, stream, p);
-        else
-          return fail("Attention: contiguous caches of 4 GiB or more are not supported.");
+        if (mode == 0) TMC_ATTN(0, kWideWaves);
+        else if (mode == 1) TMC_ATTN(1, kWideWaves);
+        else TMC_ATTN(2, kWideWaves);
       } else {
         return fail("Attention: internal error (wide blocks for a large GQA group).");
       }
     } else if (p.waves == kMidWaves) {
       if constexpr (GROUP == 1) {
-        const dim3 block(kMidWaves * kWave);
-        if (p.kv_bytes != 0 && !PAGED)
-          hipLaunchKernelGGL((attn_mfma_kernel<1, 0, kMidWaves>), grid, block, 0, stream, p);
-        else if (p.kv_bytes != 0 && p.page_size % 16 == 0)
-          hipLaunchKernelGGL((attn_mfma_kernel<1, 1, kMidWaves>), grid, block, 0, stream, p);
-        else if (PAGED)
-          hipLaunchKernelGGL((attn_mfma_kernel<1, 2, kMidWaves>), grid, block, 0, stream, p);
-        else
-          return fail("Attention: contiguous caches of 4 GiB or more are not supported.");
+        if (mode == 0) TMC_ATTN(0, kMidWaves);
+        else if (mode == 1) TMC_ATTN(1, kMidWaves);
+        else TMC_ATTN(2, kMidWaves);
       } else {
         return fail("Attention: internal error (8-wave blocks for a GQA group).");
       }
-    } else if (p.kv_bytes != 0 && !PAGED)
-      hipLaunchKernelGGL((attn_mfma_kernel<GROUP, 0, kWaves>), grid, dim3(kThreads), 0, stream, p);
-    else if (p.kv_bytes != 0 && p.page_size % 16 == 0)
-      hipLaunchKernelGGL((attn_mfma_kernel<GROUP, 1, kWaves>), grid, dim3(kThreads), 0, stream, p);
-    else if (PAGED)
-      hipLaunchKernelGGL((attn_mfma_kernel<GROUP, 2, kWaves>), grid, dim3(kThreads), 0, stream, p);
-    else
-      return fail("Attention: contiguous caches of 4 GiB or more are not supported.");
+    } else if (mode == 0) {
+      TMC_ATTN(0, kWaves);
+    } else if (mode == 1) {
+      TMC_ATTN(1, kWaves);
+    } else {
+      TMC_ATTN(2, kWaves);
+    }
   } else {
     hipLaunchKernelGGL((attn_partial_kernel<D, GROUP, PAGED>), grid, dim3(kThreads), 0, stream, p);
   }
+#undef TMC_ATTN
   if (check_launch("attention kernel")) return 1;
   if (p.max_splits > 1 && !p.arrivals) {  // else merged in the partial kernel
     hipLaunchKernelGGL((attn_combine_kernel<D, PAGED>),
@@ -1167,6 +1210,7 @@ constexpr int kWideMaxRows = 256;
 struct SplitPlan {
   int chunk;
   int waves;
+  bool valu;
 };
 
 SplitPlan split_plan(int64_t head_dim, int64_t batch, int64_t q_heads, int64_t kv_heads,
@@ -1174,10 +1218,31 @@ SplitPlan split_plan(int64_t head_dim, int64_t batch, int64_t q_heads, int64_t k
   const int chunk = chunk_for(head_dim, batch, kv_heads, capacity);
   if (head_dim == 128 && chunk > 0 && capacity <= kMfmaMaxChunk &&
       batch * kv_heads <= kWideMaxRows && q_heads / kv_heads <= kWideMaxGroup)
-    return {(int)((capacity + kMfmaStep - 1) / kMfmaStep * kMfmaStep), kWideWaves};
+    return {(int)((capacity + kMfmaStep - 1) / kMfmaStep * kMfmaStep), kWideWaves, false};
   if (head_dim == 128 && chunk >= capacity && q_heads == kv_heads)
-    return {chunk, kMidWaves};
-  return {chunk, kWaves};
+    return {chunk, kMidWaves, false};
+  return {chunk, kWaves, head_dim < 128};
+}
+
+// The plan a launch runs: at D = 64 over whole rows (a contiguous cache below
+// 4 GiB, or pages of a multiple of 16 positions in pools below it) the MFMA
+// kernel where it is faster than the VALU kernel, never with more splits than
+// the workspace is sized for.  MI355X, random pages, VALU against MFMA: GQA 4
+// batch 24, 100-2000 positions 27.6 against 18.9 us, batch 64, 200-1500 41.0
+// against 30.7, batch 1 at 4000 12.3 against 9.9; GQA 8 batch 64, 100-2000
+// 62.1 against 24.5; one-split MHA batch 1 at 300 7.3 against 5.4, batch 8,
+// 100-900 12.9 against 10.9.  Elsewhere MHA and GQA 2 are as fast or faster
+// on VALU (batch 24 MHA, 50-250: 9.4 against 13.7; GQA 2 batch 64, 100-600
+// 27.0 against 27.2), and so are other page sizes (12: 27.9 against 28.6).
+SplitPlan launch_plan(int64_t head_dim, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                      int64_t capacity, bool whole_rows) {
+  const SplitPlan plan = split_plan(head_dim, batch, q_heads, kv_heads, capacity);
+  if (head_dim != 64 || !whole_rows) return plan;
+  if (q_heads / kv_heads > kWideMaxGroup)
+    return {batch * kv_heads * capacity / 256 >= 1024 ? 2 * plan.chunk : plan.chunk, kWaves, false};
+  if (capacity <= kMfmaMaxChunk && batch * kv_heads <= kWideMaxRows)
+    return {(int)((capacity + kMfmaStep - 1) / kMfmaStep * kMfmaStep), kWideWaves, false};
+  return plan;
 }
 
 template <bool PAGED>
@@ -1281,9 +1346,11 @@ extern "C" int tmc_decode_attention(const void* q, const void* key_cache, const 
     const uint64_t bytes = (uint64_t)batch * kv_heads * capacity * head_dim * 2;
     p.kv_bytes = bytes < kAbsent ? (unsigned)bytes : 0u;
   }
-  const SplitPlan plan = split_plan(head_dim, batch, q_heads, kv_heads, capacity);
+  const SplitPlan plan =
+      launch_plan(head_dim, batch, q_heads, kv_heads, capacity, p.kv_bytes != 0);
   p.chunk = plan.chunk;
   p.waves = plan.waves;
+  p.valu = plan.valu;
   p.max_splits = (int)((capacity + p.chunk - 1) / p.chunk);
   p.scale_log2 = (float)(1.0 / std::sqrt((double)head_dim)) * 1.4426950408889634f;
   return dispatch_attention<false>(p, (int)batch, (int)head_dim, as_stream(stream));
@@ -1339,9 +1406,11 @@ int paged_attention_impl(const void* q, const void* key_pool, const void* value_
     p.kv_bytes = pool_pages > 0 && bytes < kAbsent ? (unsigned)bytes : 0u;
   }
   p.max_pages = (int)max_pages;
-  const SplitPlan plan = split_plan(head_dim, max_batch, q_heads, kv_heads, capacity);
+  const SplitPlan plan = launch_plan(head_dim, max_batch, q_heads, kv_heads, capacity,
+                                     p.kv_bytes != 0 && page_size % 16 == 0);
   p.chunk = plan.chunk;
   p.waves = plan.waves;
+  p.valu = plan.valu;
   p.max_splits = (int)((capacity + p.chunk - 1) / p.chunk);
   p.scale_log2 = (float)(1.0 / std::sqrt((double)head_dim)) * 1.4426950408889634f;
   return dispatch_attention<true>(p, (int)max_batch, (int)head_dim, as_stream(stream));
@@ -1689,9 +1758,9 @@ __global__ __launch_bounds__(kAoWaves * kWave) void attn_out_kernel(AttnOutParam
       const __amdgpu_buffer_rsrc_t rv = buffer_of(p.v, p.kv_bytes);
       float (*s_pw)[GROUP] = s_p[wave];
       for (int p0 = kMfmaStep * wave; p0 < valid; p0 += kMfmaStep * WAVES) {
-        KvStep<1> st;
-        issue_step<1>(p, s_pages, 0, 0, kvh, p0, valid, j, g, rk, rv, st);
-        consume_step<GROUP, 1>(p, s_pages, 0, st, qb, p0, valid, j, g, s_pw, m, lsum, o);
+        KvStep<D, 1> st;
+        issue_step<D, 1>(p, s_pages, 0, 0, kvh, p0, valid, j, g, rk, rv, st);
+        consume_step<D, GROUP, 1>(p, s_pages, 0, st, qb, p0, valid, j, g, s_pw, m, lsum, o);
       }
     }
 #pragma unroll

@@ -1,0 +1,91 @@
+"""Decode attention at head dim 64: the MFMA kernel (GQA 4 and 8, and one-split
+rows of MHA and GQA 2) and the VALU kernel beside it, at the edges of their
+splits, steps and pages, against 64-bit attention.  Tolerance: both hold the
+weights in fp32 (the MFMA form as two fp16 parts), so outputs, weighted means
+of N(0, 1) values, are off by their fp16 rounding (2^-11 of at most 5) and
+fp32 sums."""
+import math
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 5 * 2 ** -11 + 2 ** -12
+
+
+def _ref(torch, q, k, v):
+    """q [heads, d], k / v [positions, kv_heads, d]."""
+    group = q.shape[0] // k.shape[1]
+    out = []
+    for h in range(q.shape[0]):
+        kh, vh = k[:, h // group].double().contiguous(), v[:, h // group].double().contiguous()
+        out.append(torch.softmax(kh @ q[h].double() / math.sqrt(q.shape[1]), 0) @ vh)
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("qh,kvh,p,lengths,capacity,sharp", [
+    (8, 2, 16, [1, 15, 16, 17, 31, 33, 127, 129], 256, 1),
+    (16, 2, 16, [1, 255, 256, 257, 600, 1000], 1024, 1), (32, 8, 16, [2047, 5, 1300] * 8, 2048, 30),
+    (8, 1, 48, [700, 47, 49, 95], 960, 30), (4, 4, 16, [1, 32, 511, 512, 513, 1023], 1024, 1),
+    (8, 4, 32, [900, 3, 33], 1024, 30), (32, 32, 16, [300] * 9 + [1], 512, 1),
+    (8, 2, 12, [500, 11, 12, 13], 504, 1), (4, 4, 16, [1500, 20], 2048, 1)])
+def test_paged_d64_matches_fp64(tmc, qh, kvh, p, lengths, capacity, sharp):
+    import torch
+    torch.manual_seed(qh * 100 + p)
+    d, b, max_pages = 64, len(lengths), capacity // p
+    need = [-(-n // p) for n in lengths]
+    pages = sum(need) + 2
+    order = torch.randperm(pages)
+    table = torch.full((b, max_pages), -1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = order[at:at + n].int()
+        at += n
+    k, v = (torch.randn((pages, kvh, p, d), device="cuda").half() for _ in range(2))
+    k *= sharp ** 0.5
+    q = torch.randn((b, qh * d), device="cuda").half() * sharp ** 0.5
+    out = torch.full_like(q, float("nan"))
+    ws = torch.zeros(max(tmc.attention_workspace_bytes(b, qh, kvh, d, capacity) // 4, 1),
+                     dtype=torch.float32, device="cuda")
+    i32 = lambda x: torch.as_tensor(x, dtype=torch.int32).cuda()  # noqa: E731
+    args = (q, k, v, i32(lengths), i32(table), i32([b]))
+    tmc.paged_decode_attention(*args, out, b, qh, kvh, d, p, max_pages, kvh * p * d, p * d, ws)
+    for i, n in enumerate(lengths):
+        rows = table[i, :need[i]].long().cuda()
+        flat = [t[rows].permute(0, 2, 1, 3).reshape(-1, kvh, d)[:n] for t in (k, v)]
+        err = (out[i].view(qh, d).double() - _ref(torch, q[i].view(qh, d), *flat)).abs().max().item()
+        assert err <= TOL, (i, n, err)
+    # a missing page leaves its row's output untouched, the others as they were
+    hit = max(range(b), key=lambda i: need[i])
+    table[hit, need[hit] // 2] = -1
+    again = torch.full_like(q, float("nan"))
+    tmc.paged_decode_attention(*args[:4], i32(table), args[5], again, b, qh, kvh, d, p, max_pages,
+                               kvh * p * d, p * d, ws)
+    assert bool(torch.isnan(again[hit]).all())
+    keep = [i for i in range(b) if i != hit]
+    assert torch.equal(again[keep], out[keep])
+
+
+@pytest.mark.parametrize("b,qh,kvh,capacity,length", [
+    (1, 8, 2, 2048, 2047), (1, 32, 8, 4096, 1025), (2, 8, 1, 512, 31), (1, 8, 8, 1024, 900),
+    (1, 4, 4, 2000, 1999),
+    (64, 32, 32, 16384, 300)])  # 4 GiB a cache: past the buffer loads' range
+def test_contiguous_d64_matches_fp64(tmc, b, qh, kvh, capacity, length):
+    import torch
+    torch.manual_seed(capacity + length)
+    d = 64
+    k = torch.zeros((b, kvh, capacity, d), dtype=torch.float16, device="cuda")
+    v = torch.zeros_like(k)
+    for t in (k, v):
+        t[:, :, :length] = torch.randn((b, kvh, length, d), device="cuda").half()
+    q = torch.randn((b, qh * d), device="cuda").half()
+    out = torch.full_like(q, float("nan"))
+    ws = torch.zeros(max(tmc.attention_workspace_bytes(b, qh, kvh, d, capacity) // 4, 1),
+                     dtype=torch.float32, device="cuda")
+    tmc.decode_attention(q, k, v, torch.tensor([length], dtype=torch.int32, device="cuda"), out, b,
+                         qh, kvh, d, capacity, ws)
+    for i in sorted({0, b - 1}):
+        ref = _ref(torch, q[i].view(qh, d), k[i, :, :length].transpose(0, 1),
+                   v[i, :, :length].transpose(0, 1))
+        err = (out[i].view(qh, d).double() - ref).abs().max().item()
+        assert err <= TOL, (i, err)
