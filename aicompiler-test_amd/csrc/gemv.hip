@@ -30,6 +30,7 @@
 // runs either algorithm over the Wg and Wu rows of each feature and finishes
 // with the reference rounding points h(h(silu(h(g))) * h(u)).
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 #include "tmc_abi.hpp"
@@ -607,98 +608,128 @@ __device__ __forceinline__ h8 rsrc_h8(__amdgpu_buffer_rsrc_t r, unsigned byte_of
   return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte_offset, 0, 0));
 }
 
-// Block = KS waves over RT tiles of 16 output rows; wave ks takes a
-// contiguous run of K tiles (128 k), U adjacent tiles per round trip.  Lane (j = l % 16,
-// g = l / 16): A = activations (batch row j, k chunk 4s+g of the tile), B =
-// weights (output row j of the tile, same k chunk); acc[r] = out[batch
-// 4g + r][row j].
-template <int MATS, int RT, int U, typename OutT>
-__global__ __launch_bounds__(1024) void mfma_rows_kernel(const half_t* __restrict__ x,
-                                                        const half_t* __restrict__ w0,
-                                                        const half_t* __restrict__ w1,
-                                                        OutT* __restrict__ y, int m_rows,
-                                                        int n_out, int k_in, int ks_count) {
-  extern __shared__ float red[];  // [ks][MATS][RT][4][64]
+// Block = KS waves over `block_rows` (at most 16 RT) output rows; wave ks
+// takes a contiguous run of K tiles (128 k), U adjacent tiles per round trip.
+// Lane (j = l % 16, g = l / 16): A = activations (batch row 16 mt + j, k chunk
+// 4s+g of the tile), B = weights (output row j of a 16-row tile, same k
+// chunk); acc[r] = out[batch 16 mt + 4g + r][row j].
+//
+// A weight load reads 4 whole 256-byte rows of a tile (8 full cache lines)
+// and the tile is re-laid in the operand order through the wave's own LDS
+// slices (chunk c of row r at slot c ^ r); read in the operand order, a load
+// touches 16 rows x 64 bytes, half lines of 16 DRAM rows.  MI355X, weights
+// beyond the caches: 8 x 4096 x 4096 9.3 -> 7.7 us, 8 x 4096 x 12288 26.9 ->
+// 19.6, gate/up 8 x 4096 x 11008 41.3 -> 31.6 (5.7 TB/s).  More tiles in
+// flight per wave (U) no longer help.
+template <int MATS, int RT, int MT, int U, int THREADS, typename OutT>
+__global__ __launch_bounds__(THREADS) void mfma_rows_kernel(
+    const half_t* __restrict__ x, const half_t* __restrict__ w0, const half_t* __restrict__ w1,
+    OutT* __restrict__ y, int m_rows, int n_out, int k_in, int ks_count, int block_rows) {
+  extern __shared__ __attribute__((aligned(16))) float red[];  // [ks][MATS][RT][MT][4][64]
   const int lane = threadIdx.x & (kWave - 1);
   const int ks = threadIdx.x / kWave;
   const int j = lane & 15;
   const int g = lane >> 4;
-  const int n0 = blockIdx.x * RT * 16;
+  const int n0 = blockIdx.x * block_rows;
+  const int n_end = min(n_out, n0 + block_rows);
   const unsigned x_bytes = (unsigned)m_rows * (unsigned)k_in * 2u;
   const unsigned w_bytes = (unsigned)n_out * (unsigned)k_in * 2u;
   const __amdgpu_buffer_rsrc_t rx = rsrc_of(x, x_bytes);
   const __amdgpu_buffer_rsrc_t rw0 = rsrc_of(w0, w_bytes);
   const __amdgpu_buffer_rsrc_t rw1 = rsrc_of(MATS == 2 ? w1 : w0, w_bytes);
-  const unsigned x_row = j < m_rows ? (unsigned)j * (unsigned)k_in * 2u : kNoData;
-  unsigned w_row[RT];
+  unsigned x_row[MT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int row = n0 + rt * 16 + j;
-    w_row[rt] = row < n_out ? (unsigned)row * (unsigned)k_in * 2u : kNoData;
-  }
-  f4 acc[MATS][RT];
+  for (int mt = 0; mt < MT; ++mt)
+    x_row[mt] = 16 * mt + j < m_rows ? (unsigned)(16 * mt + j) * (unsigned)k_in * 2u : kNoData;
+  f4 acc[MATS][RT][MT];
 #pragma unroll
   for (int m = 0; m < MATS; ++m)
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[m][rt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[m][rt][mt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   // Wave ks owns the contiguous K tiles [first, last): the U tiles of one
   // round trip are adjacent, so each weight row is read in U*256-byte runs.
   const int tiles = (k_in + 127) / 128;
   const int per_wave = (tiles + ks_count - 1) / ks_count;
   const int first = ks * per_wave;
   const int last = min(tiles, first + per_wave);
+  h8* slices = reinterpret_cast<h8*>(red) + ks * 512;
   for (int t0 = first; t0 < last; t0 += U) {
-    h8 xv[U][4], wv[U][MATS][RT][4];
+    h8 xv[U][MT][4], wv[U][MATS][RT][4];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int k = (t0 + u) * 128 + 32 * s + 8 * g;
-        const bool kok = t0 + u < last && k < k_in;
-        const unsigned kb = (unsigned)k * 2u;
-        xv[u][s] = rsrc_h8(rx, kok && x_row != kNoData ? x_row + kb : kNoData);
+        const bool live = t0 + u < last;
+        const bool kok = live && k < k_in;
         // default cache policy for the weights: the non-temporal hint
         // measured slower here (C2 at batch 8, row-major: 3.90 -> 3.71 TB/s)
+        const int wk = (t0 + u) * 128 + 8 * j;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-          const unsigned off = kok && w_row[rt] != kNoData ? w_row[rt] + kb : kNoData;
+          const int row = n0 + rt * 16 + 4 * s + g;
+          const unsigned off = live && wk < k_in && row < n_end
+                                   ? (unsigned)row * (unsigned)k_in * 2u + (unsigned)wk * 2u
+                                   : kNoData;
           wv[u][0][rt][s] = rsrc_h8(rw0, off);
           if constexpr (MATS == 2) wv[u][1][rt][s] = rsrc_h8(rw1, off);
         }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          xv[u][mt][s] =
+              rsrc_h8(rx, kok && x_row[mt] != kNoData ? x_row[mt] + (unsigned)k * 2u : kNoData);
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int m = 0; m < MATS; ++m)
 #pragma unroll
-        for (int m = 0; m < MATS; ++m)
+        for (int rt = 0; rt < RT; ++rt) {
+          h8 wf[4];
+          h8* slice = slices + 256 * ((u * MATS * RT + m * RT + rt) & 1);
 #pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
-            acc[m][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[u][s], wv[u][m][rt][s],
-                                                                acc[m][rt], 0, 0, 0);
+          for (int s = 0; s < 4; ++s) slice[(4 * s + g) * 16 + (j ^ (4 * s + g))] = wv[u][m][rt][s];
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int s = 0; s < 4; ++s) wf[s] = slice[j * 16 + ((4 * s + g) ^ j)];
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+              acc[m][rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[u][mt][s], wf[s],
+                                                                      acc[m][rt][mt], 0, 0, 0);
+        }
   }
-  constexpr int kValues = MATS * RT * 4;  // per lane
+  __syncthreads();  // the slices become the sums
+  constexpr int kValues = MATS * RT * MT * 4;  // per lane
 #pragma unroll
   for (int m = 0; m < MATS; ++m)
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        red[((size_t)ks * kValues + (m * RT + rt) * 4 + r) * kWave + lane] = acc[m][rt][r];
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          red[((size_t)ks * kValues + ((m * RT + rt) * MT + mt) * 4 + r) * kWave + lane] =
+              acc[m][rt][mt][r];
   __syncthreads();
-  // Every thread finishes some (rt, r, lane) outputs: sum the KS partials.
-  const int total = RT * 4 * kWave;
+  // Every thread finishes some (rt, mt, r, lane) outputs: sum the KS partials.
+  const int total = RT * MT * 4 * kWave;
   for (int idx = threadIdx.x; idx < total; idx += ks_count * kWave) {
-    const int l = idx % kWave, rt = (idx / kWave) / 4, r = (idx / kWave) % 4;
+    const int l = idx % kWave, v = idx / kWave;  // v = (rt MT + mt) 4 + r
+    const int rt = v / (4 * MT), mt = v / 4 % MT, r = v % 4;
     float a[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
       for (int w = 0; w < ks_count; ++w)
-        a[m] += red[((size_t)w * kValues + (m * RT + rt) * 4 + r) * kWave + l];
-    const int row = 4 * (l >> 4) + r;       // batch row
-    const int col = n0 + rt * 16 + (l & 15);  // output feature
-    if (row < m_rows && col < n_out) write_out<MATS>(y, (size_t)row * n_out + col, a[0], a[1]);
+        a[m] += red[((size_t)w * kValues + m * RT * MT * 4 + v) * kWave + l];
+    const int row = 16 * mt + 4 * (l >> 4) + r;  // batch row
+    const int col = n0 + rt * 16 + (l & 15);     // output feature
+    if (row < m_rows && col < n_end) write_out<MATS>(y, (size_t)row * n_out + col, a[0], a[1]);
   }
 }
 
@@ -884,12 +915,14 @@ int run_mfma(const Shape& s, const tmc_gemv_config& cfg, hipStream_t st) {
   return 0;
 }
 
-template <int MATS, int RT, int U, typename OutT>
-int launch_rows(const Shape& s, const half_t* x, OutT* y, int rows, int ks, hipStream_t st) {
-  const dim3 grid((unsigned)((s.n + RT * 16 - 1) / (RT * 16)));
-  const size_t lds = (size_t)ks * MATS * RT * 4 * kWave * sizeof(float);
-  hipLaunchKernelGGL((mfma_rows_kernel<MATS, RT, U, OutT>), grid, dim3(ks * kWave), lds, st, x,
-                     s.w0, s.w1, y, rows, s.n, s.k, ks);
+template <int MATS, int RT, int MT, int U, int THREADS, typename OutT>
+int launch_rows(const Shape& s, const half_t* x, OutT* y, int rows, int ks, int block_rows,
+                hipStream_t st) {
+  const dim3 grid((unsigned)((s.n + block_rows - 1) / block_rows));
+  const size_t sums = (size_t)ks * MATS * RT * MT * 4 * kWave * sizeof(float);
+  const size_t lds = std::max(sums, (size_t)ks * 512 * sizeof(h8));  // or the waves' slices
+  hipLaunchKernelGGL((mfma_rows_kernel<MATS, RT, MT, U, THREADS, OutT>), grid, dim3(ks * kWave), lds, st, x,
+                     s.w0, s.w1, y, rows, s.n, s.k, ks, block_rows);
   return check_launch("mfma_rows_kernel");
 }
 
@@ -905,16 +938,76 @@ int run_rows(const Shape& s, const tmc_gemv_config& cfg, hipStream_t st) {
     OutT* ys = y + (size_t)r0 * s.n;
     int rc;
     const int ks = cfg.k_split;
+    // 16 waves leave a lane 128 registers, 8 waves 256
+#define TMC_ROWS(RT, U)                                                                          \
+  rc = ks <= 8 ? launch_rows<MATS, RT, 1, U, 512, OutT>(s, xs, ys, rows, ks, 16 * RT, st)        \
+               : launch_rows<MATS, RT, 1, U, 1024, OutT>(s, xs, ys, rows, ks, 16 * RT, st)
     switch (cfg.rows_per_wave * 8 + cfg.unroll) {
-    case 9: rc = launch_rows<MATS, 1, 1, OutT>(s, xs, ys, rows, ks, st); break;
-    case 10: rc = launch_rows<MATS, 1, 2, OutT>(s, xs, ys, rows, ks, st); break;
-    case 12: rc = launch_rows<MATS, 1, 4, OutT>(s, xs, ys, rows, ks, st); break;
-    case 17: rc = launch_rows<MATS, 2, 1, OutT>(s, xs, ys, rows, ks, st); break;
-    case 18: rc = launch_rows<MATS, 2, 2, OutT>(s, xs, ys, rows, ks, st); break;
-    case 20: rc = launch_rows<MATS, 2, 4, OutT>(s, xs, ys, rows, ks, st); break;
-    case 33: rc = launch_rows<MATS, 4, 1, OutT>(s, xs, ys, rows, ks, st); break;
-    default: rc = launch_rows<MATS, 4, 2, OutT>(s, xs, ys, rows, ks, st); break;
+    case 9: TMC_ROWS(1, 1); break;
+    case 10: TMC_ROWS(1, 2); break;
+    case 12: TMC_ROWS(1, 4); break;
+    case 17: TMC_ROWS(2, 1); break;
+    case 18: TMC_ROWS(2, 2); break;
+    case 20: TMC_ROWS(2, 4); break;
+    case 33: TMC_ROWS(4, 1); break;
+    default: TMC_ROWS(4, 2); break;
     }
+#undef TMC_ROWS
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+// The row-tile kernel as the default picks it: up to 64 batch rows per launch
+// (weights read once), and blocks of equal height that fill whole rounds of
+// the 256 CUs.  Of one to four rounds with at most 48 rows a block, the one
+// that reads least per CU (its weight rows and the batch rows beside them);
+// a single round takes 8 waves per block, several rounds 4, whose blocks
+// share a CU.  7 x 4104 x 5003: 251 blocks of 20 rows 9.9 us, 313 of 16 (57
+// CUs with two) 13; 16 x 4096 x 12288: 256 blocks of 48 rows 20.6 us, 768 of
+// 16 22.4; 30 x 4104 x 5003 in one launch of 32 rows 14.5 us, 37.0 in two of
+// 16 before.
+template <int MATS, typename OutT>
+int run_rows_default(const Shape& s, hipStream_t st) {
+  OutT* y = static_cast<OutT*>(s.y);
+  const int tiles = (int)std::min<int64_t>(4, ((int64_t)s.batch + 15) / 16);
+  int block_rows = 16, best = INT_MAX, rounds = (s.n + 4095) / 4096;
+  for (int r = 1; r <= 4; ++r) {
+    const int rows = std::max(8, (s.n + 256 * r - 1) / (256 * r));
+    const int cost = r * (MATS * rows + 16 * tiles);
+    // (48 rows of two matrices beside 64 batch rows would spill)
+    const int most = MATS == 2 && tiles == 4 ? 32 : 48;
+    if (rows <= most && cost < best) {
+      best = cost;
+      block_rows = rows;
+      rounds = r;
+    }
+  }
+  const int rt = (block_rows + 15) / 16;
+  const int ks = rounds == 1 && rt * MATS <= 2 ? 8 : 4;
+  for (int64_t r0 = 0; r0 < s.batch; r0 += 16 * tiles) {
+    const int rows = (int)std::min<int64_t>(16 * tiles, s.batch - r0);
+    const half_t* xs = s.x + (size_t)r0 * s.k;
+    OutT* ys = y + (size_t)r0 * s.n;
+    int rc = 0;
+#define TMC_ROWS_MT(RT, MT)                                                                      \
+  rc = launch_rows<MATS, RT, MT, 1, 512, OutT>(s, xs, ys, rows, ks, block_rows, st)
+#define TMC_ROWS(RT)                                                                             \
+  switch ((rows + 15) / 16) {                                                                    \
+  case 1: TMC_ROWS_MT(RT, 1); break;                                                             \
+  case 2: TMC_ROWS_MT(RT, 2); break;                                                             \
+  case 3: TMC_ROWS_MT(RT, 3); break;                                                             \
+  default: TMC_ROWS_MT(RT, 4); break;                                                            \
+  }
+    if (rt == 1) {
+      TMC_ROWS(1)
+    } else if (rt == 2) {
+      TMC_ROWS(2)
+    } else {
+      TMC_ROWS(3)
+    }
+#undef TMC_ROWS
+#undef TMC_ROWS_MT
     if (rc) return rc;
   }
   return 0;
@@ -1069,8 +1162,14 @@ int run_linear(int mats, const void* x, const void* w0, const void* w1, void* y,
   }
   if (cfg.algorithm == 3) {
     // raw buffers address at most 4 GiB - 16 bytes
-    const uint64_t wb = (uint64_t)s.n * s.k * 2, xb = (uint64_t)min(s.batch, 16) * s.k * 2;
-    if (wb < kNoData && xb < kNoData) {
+    const uint64_t wb = (uint64_t)s.n * s.k * 2, xb = (uint64_t)min(s.batch, 64) * s.k * 2;
+    const bool chosen = user && user->algorithm != 0;
+    if (wb < kNoData && xb < kNoData && !chosen) {
+      if (mats == 2) return run_rows_default<2, half_t>(s, st);
+      return y_dtype == TMC_F32 ? run_rows_default<1, float>(s, st)
+                                : run_rows_default<1, half_t>(s, st);
+    }
+    if (wb < kNoData && (uint64_t)min(s.batch, 16) * s.k * 2 < kNoData) {
       if (mats == 2) return run_rows<2, half_t>(s, cfg, st);
       return y_dtype == TMC_F32 ? run_rows<1, float>(s, cfg, st) : run_rows<1, half_t>(s, cfg, st);
     }
