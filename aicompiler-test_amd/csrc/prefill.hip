@@ -357,14 +357,15 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
 // store.  Rows are swizzled in 16-byte chunks (K) and 32-byte units (V) so
 // that operand reads spread over the banks.
 //
-// Softmax per wave over its own positions: weights 2^(s - m) with m raised
-// only when a score passes it by more than 8 (so they stay below 2^8 and the
-// outputs are seldom rescaled); their sum is one more MFMA over the rounded
-// weights.  The position groups meet in LDS at the end.
+// Softmax per wave over its own positions: weights 2^(s - m) with m their
+// running maximum (a tile without a new one skips the rescale); their sum is
+// one more MFMA over the rounded weights.  The position groups meet in LDS at
+// the end.
 //
-// MI355X, against the 16-vector kernel: 512 tokens at 3584 (GQA 4) 105 -> 48
-// us, 2048 tokens (MHA) 96 -> 68 (510 TFLOP/s), head dim 64, 1024 at 1024
-// 50 -> 27.  What bounds it now is the softmax's VALU work beside the MFMAs,
+// MI355X, against the 16-vector kernel: 512 tokens at 3584 (GQA 4) 105 -> 56
+// us, 2048 tokens (MHA) 96 -> 74 (470 TFLOP/s), head dim 64, 1024 at 1024
+// 50 -> 31.  Error against 64 bits over contexts of 2000 to 4096: 2.75e-4 of
+// the rms, 2.82e-4 before (2.07e-4 of it the output's rounding).  What bounds it now is the softmax's VALU work beside the MFMAs,
 // and for few blocks the latency of one block's loads.
 constexpr size_t kPtTable = 28 * 1024;  // block-table bytes beside 128 KiB of buffers
 
@@ -584,23 +585,18 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
           for (int r = 0; r < 4; ++r)
             if (first + 16 * t + 4 * g + r >= len[v]) sc[v][t][r] = -INFINITY;
     }
-    float next[2];
-    bool raise = false;
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
       float b = fmaxf(fmaxf(fmaxf(sc[v][0][0], sc[v][0][1]), fmaxf(sc[v][0][2], sc[v][0][3])),
                       fmaxf(fmaxf(sc[v][1][0], sc[v][1][1]), fmaxf(sc[v][1][2], sc[v][1][3])));
       b = max_over_groups(b) * p.scale_log2;
-      // the first finite score, or one that passes m by more than 2^8
-      const bool up = b > m[v] + 8.0f;
-      next[v] = up ? b : m[v];
-      raise = raise || up;
-    }
-    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
-#pragma unroll
-      for (int v = 0; v < 2; ++v) {
-        const float alpha = next[v] == m[v] ? 1.0f : fast_exp2(m[v] - next[v]);
-        m[v] = next[v];
+      // The running maximum is followed exactly: its weight is then 1 and the
+      // greatest weights lie just below it, where fp16 rounds them best.  A
+      // maximum that lagged by up to 2^8 rounded them 6% worse.
+      if (__builtin_amdgcn_ballot_w64(b > m[v]) != 0) {
+        const float next = fmaxf(m[v], b);
+        const float alpha = next == m[v] ? 1.0f : fast_exp2(m[v] - next);
+        m[v] = next;
         lsum[v] *= alpha;
 #pragma unroll
         for (int t = 0; t < DT; ++t) o[v][t] *= alpha;
@@ -774,10 +770,10 @@ extern "C" int tmc_prefill_attention_rows_f16(const void* q, const void* key_poo
   if (buf && rows16 && table_lds <= kPtTable) {
     // Four position groups (8 waves, 128 positions a block) where a launch has
     // at most one block per CU and contexts may be long: 512 tokens at 3584,
-    // GQA 4: 48 us against 63 with two groups, 16 at 3000 37 against 49; with
+    // GQA 4: 56 us against 72 with two groups, 16 at 3000 43 against 56; with
     // more blocks than CUs two 4-wave blocks share a CU and two groups win
-    // (2048 tokens MHA 68 against 75), and below about 500 positions the
-    // longer hand-over costs more than it saves (200 tokens 8.8 against 10.2).
+    // (2048 tokens MHA 74 against 83), and below about 500 positions the
+    // longer hand-over costs more than it saves (200 tokens 9.2 against 10.6).
     const bool four = grid.x <= 256 && page_size * max_pages > 1024;
 #define TMC_PT_LAUNCH(DIM, PG) \
   hipLaunchKernelGGL((prefill_tile_kernel<DIM, PG>), grid, dim3(2 * PG * kWave), table_lds, s, p)
