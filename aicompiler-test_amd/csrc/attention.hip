@@ -1105,7 +1105,7 @@ int launch_group(const AttnParams& params, int batch, hipStream_t stream) {
   hipLaunchKernelGGL((attn_mfma_kernel<D, GROUP, MODE, WAVES>), grid, dim3(WAVES * kWave), 0,    \
                      stream, p)
   if constexpr (D == 64) {
-    // split_plan: whole-row forms only, wide blocks of groups up to 2 and
+    // launch_plan: whole-row forms only, wide blocks of groups up to 2 and
     // 4-wave blocks of wider ones
     if (p.valu) {
       hipLaunchKernelGGL((attn_partial_kernel<D, GROUP, PAGED>), grid, dim3(kThreads), 0, stream, p);

@@ -164,9 +164,12 @@ void tmc_exec_release(tmc_exec *exec);
 /* MetalRuntime::prepareSequence / PreparedSequence::execute
  * (MetalRuntime.hpp:130-142,202-203; .mm:292-341,751-781): the steps are
  * captured once into a HIP graph and replayed with one hipGraphLaunch.  A
- * sequence that holds a step kept out of graphs replays its steps eagerly,
- * in order, on the runtime's stream instead.  Either way the steps and their
- * buffers must outlive the sequence. */
+ * sequence that holds a step kept out of graphs, or whose graph has at most
+ * six nodes (their launches cost less than the graph's), queues its steps'
+ * launches in order on the runtime's stream instead; the small graph is still
+ * what is launched while that stream is being captured.  Either way the steps
+ * and their buffers must outlive the sequence, and what other threads queue on
+ * the runtime falls before or after the whole replay. */
 int tmc_seq_create(tmc_runtime *rt, tmc_exec *const *steps, size_t n, tmc_seq **out);
 int tmc_seq_run(tmc_seq *seq, double *gpu_us, double *cpu_us);
 /* Enqueue one replay on the runtime stream without waiting. */
