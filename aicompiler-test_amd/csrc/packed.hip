@@ -437,10 +437,14 @@ int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int
     const int rows = (int)std::min<int64_t>(16 * tiles, batch - r0);
     const int mt = (rows + 15) / 16;
     const int nt = FUSE == kPackedResidual ? 1 : column_tiles(mt, n, MATS);
-    if (nt > 1) ks = 8;
+    // of this pass alone: the last one may hold fewer row tiles, and then one
+    // column tile, whose norm form is built for kPackedNormWaves waves
+    const int waves = nt > 1 ? 8 : ks;
+    TMC_REQUIRE(waves * kWave <= packed_threads(MATS, nt, mt, FUSE),
+                "Packed GEMM: internal error (more waves than the kernel's bound).");
     const dim3 grid((unsigned)(((n + 15) / 16 + nt - 1) / nt));
-    const size_t lds = (size_t)ks * MATS * mt * 4 * kWave * sizeof(float) +
-                       (FUSE == kPackedNorm ? (size_t)ks * mt * 16 * sizeof(float) : 0);
+    const size_t lds = (size_t)waves * MATS * mt * 4 * kWave * sizeof(float) +
+                       (FUSE == kPackedNorm ? (size_t)waves * mt * 16 * sizeof(float) : 0);
     const half_t* xs = x + (r0 / 16) * x_pass;
     OutT* ys = ROPE || ARGMAX ? y : y + (r0 / 16) * y_pass;
     RopeArgs ra = rope;
@@ -449,7 +453,7 @@ int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int
     if (FUSE == kPackedResidual) pf.residual = fuse.residual + (r0 / 16) * y_pass;
 #define TMC_PACKED_LAUNCH(N, M, U)                                                               \
   hipLaunchKernelGGL((packed_gemm_kernel<MATS, N, M, U, OutT, XP, YP, ROPE, FUSE, ARGMAX>), grid,   \
-                     dim3(ks * kWave), lds, st, xs, p0, p1, ys, rows, (int)n, (int)k, ks,        \
+                     dim3(waves * kWave), lds, st, xs, p0, p1, ys, rows, (int)n, (int)k, waves,  \
                      (unsigned)bytes, ra, pf)
     if (nt == 3) {
       if constexpr (FUSE != kPackedResidual) {

@@ -129,3 +129,76 @@ def test_qkv_rope_rows_equal_unfused(tmc, orc, torch, batch, qh):
         out.append([bits(t) for t in (q, kp, vp)])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def _norm_ref(x, w, gamma):
+    xd = x.double()
+    norm = xd / ((xd * xd).mean(-1, keepdim=True) + 1e-6).sqrt()
+    return norm @ (w.float() * gamma.float()).half().double().t()
+
+
+@pytest.mark.parametrize("batch,n", [(65, 12300), (80, 12300), (130, 12288), (70, 20000)])
+def test_norm_remainder_rows_match_fp64(tmc, orc, torch, batch, n):
+    """Folded norm, a last pass of at most 16 rows after 64-row passes with
+    three column tiles: logits and the token-only head's tokens."""
+    k = 264
+    x = dev_f16(orc.f16(normal(2041 + batch, (batch, k))))
+    gamma = dev_f16(orc.f16(uniform(2042, (k,), 0.5, 1.5)))
+    w = dev_f16(orc.f16(normal(2043, (n, k), 0.02)))
+    packed, xin = tmc.pack_weights(w, gamma=gamma), tmc.pack_activations(x)
+    y = torch.full((batch, n), float("nan"), dtype=torch.float32, device="cuda")
+    tmc.gemm_packed_norm(xin, packed, y, batch, k, n, 1e-6, 1)
+    assert_f32_rel(values(y), _norm_ref(x, w, gamma).cpu().numpy(), what=f"b{batch} n{n}")
+    ws = torch.zeros(tmc.lm_head_argmax_workspace_bytes(batch, n) // 4, dtype=torch.float32,
+                     device="cuda")
+    tok = torch.full((batch,), -7, dtype=torch.int32, device="cuda")
+    tmc.lm_head_argmax_packed_norm(xin, packed, ws, tok, batch, k, n, 1e-6, 1)
+    assert torch.equal(tok.long(), y.argmax(-1))
+
+
+@pytest.mark.parametrize("batch,n", [(65, 11008), (80, 11008), (97, 9600), (112, 9600),
+                                     (96, 10400)])
+def test_gated_remainder_rows_match_fp64(tmc, orc, torch, batch, n):
+    """Gate/up: last passes of one to three row tiles with one column tile
+    after passes with three."""
+    k = 264
+    x = dev_f16(orc.f16(normal(2051 + batch, (batch, k))))
+    one = dev_f16(orc.f16(np.ones(k, np.float32)))
+    wg, wu = (dev_f16(orc.f16(normal(s, (n, k), 0.02))) for s in (2052, 2053))
+    out = torch.zeros(tmc.packed_activation_elements(batch, n), dtype=torch.float16, device="cuda")
+    tmc.gate_up_silu_packed_norm(tmc.pack_activations(x), tmc.pack_weights(wg, gamma=one),
+                                 tmc.pack_weights(wu, gamma=one), out, batch, k, n, 1e-6, 3)
+    got = torch.empty((batch, n), dtype=torch.float16, device="cuda")
+    tmc.pack_activations(out, got, unpack=True, rows=batch, cols=n)
+    g, u = _norm_ref(x, wg, one), _norm_ref(x, wu, one)
+    assert_f16_path(values(got), (g / (1 + torch.exp(-g)) * u).cpu().numpy(), what=f"b{batch}")
+
+
+@pytest.mark.parametrize("batch", [65, 80])
+def test_norm_qkv_remainder_rows_equal_their_own_call(tmc, orc, torch, batch):
+    """Fused q.k.v of 12288 columns: the 64-row pass and the remainder write
+    the bits of calls of their own, K/V pages included."""
+    qh, d, hidden, cap, p = 32, 128, 264, 64, 16
+    mp, width = cap // p, 3 * qh * d
+    rng = np.random.default_rng(2061)
+    one = dev_f16(orc.f16(np.ones(hidden, np.float32)))
+    w = tmc.pack_weights(dev_f16(orc.f16(normal(2062, (width, hidden), 0.05))), gamma=one)
+    x = dev_f16(orc.f16(normal(2063, (batch, hidden))))
+    i32 = lambda a: torch.tensor(np.asarray(a, np.int32), device="cuda")  # noqa: E731
+    ang = np.arange(cap)[:, None] * 10000.0 ** (-np.arange(0, d, 2) / d)
+    cos, sin = (torch.tensor(f(ang).astype(np.float32), device="cuda") for f in (np.cos, np.sin))
+    tables, lengths = rng.permutation(batch * mp).reshape(batch, mp), rng.integers(1, cap + 1, batch)
+    whole, parts = [], []
+    for cuts, out in (([(0, batch)], whole), ([(0, 64), (64, batch)], parts)):
+        q = torch.full((batch, qh * d), float("nan"), dtype=torch.float16, device="cuda")
+        kp = torch.zeros((batch * mp, qh, p, d), dtype=torch.float16, device="cuda")
+        vp = torch.zeros_like(kp)
+        for a, b in cuts:
+            tmc.rmsnorm_qkv_rope_append_packed(
+                tmc.pack_activations(x[a:b].contiguous()), w, cos, sin, i32(lengths[a:b]),
+                i32(tables[a:b]), i32([b - a]), q[a:b], kp, vp, b - a, hidden, qh, qh, d, cap, p,
+                mp, 1e-6, 1)
+        torch.cuda.synchronize()
+        out.extend(bits(t) for t in (q, kp, vp))
+    for a, b in zip(whole, parts):
+        assert np.array_equal(a, b)
