@@ -178,8 +178,9 @@ struct tmc_runtime {
   char* staging_device = nullptr;  // the same pinned area as the device addresses it
   size_t staged = 0;
   hipEvent_t staged_done = nullptr;
-  // Held while one call queues its work on `stream`, so that what another
-  // thread queues falls before or after all of a sequence's steps.
+  // Held while one call queues its work on `stream` (and while a sequence is
+  // captured on it), so that what another thread queues through this library
+  // falls before or after all of a sequence's steps.
   std::mutex order;
 };
 
@@ -1144,6 +1145,13 @@ extern "C" const char* tmc_rt_init_error(const tmc_runtime* rt) {
   return rt ? rt->init_error.c_str() : "null runtime";
 }
 extern "C" void* tmc_rt_stream(const tmc_runtime* rt) { return rt ? (void*)rt->stream : nullptr; }
+extern "C" int tmc_rt_enqueue(tmc_runtime* rt, int (*work)(void* stream, void* arg), void* arg) {
+  clear_error();
+  if (!rt || !work) return fail("tmc_rt_enqueue: null argument.");
+  if (!rt->available) return fail(rt->init_error);
+  const std::lock_guard<std::mutex> lock(rt->order);
+  return work((void*)rt->stream, arg);
+}
 extern "C" int tmc_rt_synchronize(tmc_runtime* rt) {
   clear_error();
   if (!rt) return fail("tmc_rt_synchronize: null runtime.");
@@ -1186,7 +1194,10 @@ extern "C" int tmc_buf_create(tmc_runtime* rt, size_t count, int dtype, const fl
     const auto host = encode(init, count, dtype);
     rc = hip_ok(hipMemcpy(buf->ptr, host.data(), bytes, hipMemcpyHostToDevice), "buffer upload");
   } else {
-    rc = fill_sentinel(buf->ptr, count, dtype, true, rt->stream);
+    {
+      const std::lock_guard<std::mutex> lock(rt->order);
+      rc = fill_sentinel(buf->ptr, count, dtype, true, rt->stream);
+    }
     if (!rc) rc = hip_ok(hipStreamSynchronize(rt->stream), "buffer fill");
   }
   if (rc) {
@@ -1313,13 +1324,16 @@ extern "C" int tmc_buf_write_raw_async(tmc_buffer* buf, const void* data, size_t
   if (!buf || !data || count == 0 || offset > buf->count || count > buf->count - offset)
     return fail("tmc_buf_write_raw_async: invalid range.");
   tmc_runtime* rt = buf->rt;
+  const size_t bytes = count * element_bytes(buf->dtype);
+  char* stage = nullptr;
+  std::unique_lock<std::mutex> lock(rt->order);
   // a captured copy would replay whatever the staging slot holds later
   if (stream_captured(rt))
     return fail("tmc_buf_write_raw_async: not allowed while the runtime stream is captured.");
-  const size_t bytes = count * element_bytes(buf->dtype);
-  if ((bytes + 255) / 256 * 256 > kStagingBytes) return tmc_buf_write_raw(buf, data, count, offset);
-  char* stage = nullptr;
-  const std::lock_guard<std::mutex> lock(rt->order);
+  if ((bytes + 255) / 256 * 256 > kStagingBytes) {
+    lock.unlock();
+    return tmc_buf_write_raw(buf, data, count, offset);
+  }
   if (stage_reserve(rt, bytes, stage)) return 1;
   std::memcpy(stage, data, bytes);
   if (hip_ok(hipMemcpyAsync(static_cast<char*>(buf->ptr) + offset * element_bytes(buf->dtype),
@@ -1343,11 +1357,11 @@ extern "C" int tmc_buf_write_sparse_async(tmc_buffer* buf, const int32_t* pairs,
       return fail("tmc_buf_write_sparse_async: indices must increase and lie inside the buffer.");
   }
   tmc_runtime* rt = buf->rt;
-  if (stream_captured(rt))
-    return fail("tmc_buf_write_sparse_async: not allowed while the runtime stream is captured.");
   const size_t bytes = count * 2 * sizeof(int32_t);
   char* stage = nullptr;
   const std::lock_guard<std::mutex> lock(rt->order);
+  if (stream_captured(rt))
+    return fail("tmc_buf_write_sparse_async: not allowed while the runtime stream is captured.");
   if (stage_reserve(rt, bytes, stage)) return 1;
   std::memcpy(stage, pairs, bytes);
   const auto* mapped = reinterpret_cast<const int32_t*>(rt->staging_device + (stage - rt->staging));
@@ -1379,10 +1393,13 @@ extern "C" int tmc_buf_read_raw(const tmc_buffer* buf, void* data, size_t count,
   if (!buf || !data || offset > buf->count || count > buf->count - offset)
     return fail("tmc_buf_read_raw: invalid range.");
   const size_t eb = element_bytes(buf->dtype);
-  if (hip_ok(hipMemcpyAsync(data, static_cast<const char*>(buf->ptr) + offset * eb, count * eb,
-                            hipMemcpyDeviceToHost, buf->rt->stream),
-             "raw read"))
-    return 1;
+  {
+    const std::lock_guard<std::mutex> lock(buf->rt->order);
+    if (hip_ok(hipMemcpyAsync(data, static_cast<const char*>(buf->ptr) + offset * eb, count * eb,
+                              hipMemcpyDeviceToHost, buf->rt->stream),
+               "raw read"))
+      return 1;
+  }
   return hip_ok(hipStreamSynchronize(buf->rt->stream), "raw read");
 }
 
@@ -1508,9 +1525,13 @@ extern "C" int tmc_prepare(tmc_runtime* rt, const tmc_kernel* kernel, tmc_buffer
     exec->ctx.workspace_bytes = s.workspace_bytes;
     // A defined starting state for the workspace (filled once, here,
     // outside any captured sequence).
-    if (hip_ok(hipMemsetAsync(exec->ctx.workspace, 0, s.workspace_bytes, rt->stream),
-               "workspace fill") ||
-        hip_ok(hipStreamSynchronize(rt->stream), "workspace fill")) {
+    int rc;
+    {
+      const std::lock_guard<std::mutex> lock(rt->order);
+      rc = hip_ok(hipMemsetAsync(exec->ctx.workspace, 0, s.workspace_bytes, rt->stream),
+                  "workspace fill");
+    }
+    if (rc || hip_ok(hipStreamSynchronize(rt->stream), "workspace fill")) {
       (void)hipFree(exec->ctx.workspace);
       return 1;
     }
@@ -1587,6 +1608,8 @@ extern "C" int tmc_seq_create(tmc_runtime* rt, tmc_exec* const* steps, size_t n,
     *out = seq.release();
     return 0;
   }
+  // another thread's work would be captured along with the steps
+  const std::lock_guard<std::mutex> lock(rt->order);
   if (hip_ok(hipStreamSynchronize(rt->stream), "sequence capture")) return 1;
   if (hip_ok(hipStreamBeginCapture(rt->stream, hipStreamCaptureModeThreadLocal), "begin capture"))
     return 1;
@@ -1614,7 +1637,9 @@ extern "C" int tmc_seq_create(tmc_runtime* rt, tmc_exec* const* steps, size_t n,
 namespace {
 // One replay of the sequence on its runtime's stream: the graph, or the
 // eager steps in order (stops at the first failing launch).  While the stream
-// is being captured a graph is launched as a graph.
+// is being captured a graph is launched as a graph.  The lock is held for both:
+// the runtime queues a graph's kernels one by one, and another thread's work
+// came between them (two threads replaying through one scratch buffer).
 int replay(tmc_seq* seq) {
   const std::lock_guard<std::mutex> lock(seq->rt->order);
   if (seq->exec && (seq->eager.empty() || stream_captured(seq->rt)))

@@ -302,10 +302,12 @@ std::string ensurePackedWeights(hip::HipRuntime& runtime, DecoderLLMModelResourc
       if (count <= 0) throw std::runtime_error("Packed weights: invalid matrix shape.");
       auto packed = allocate(runtime, static_cast<std::size_t>(count), nullptr,
                              ElementType::Float16);
-      if (tmc_pack_weights_scaled_f16(w->devicePointer(),
-                                      gamma ? (*gamma)->devicePointer() : nullptr,
-                                      packed->devicePointer(), static_cast<int64_t>(out),
-                                      static_cast<int64_t>(in), runtime.stream()) != 0)
+      if (runtime.enqueue([&](void* stream) {
+            return tmc_pack_weights_scaled_f16(w->devicePointer(),
+                                               gamma ? (*gamma)->devicePointer() : nullptr,
+                                               packed->devicePointer(), static_cast<int64_t>(out),
+                                               static_cast<int64_t>(in), stream);
+          }) != 0)
         throw std::runtime_error(std::string("Packed weights: ") + tmc_last_error());
       bytes += static_cast<std::size_t>(count) * 2;
       slot = std::move(packed);
@@ -936,12 +938,14 @@ std::string BatchedDecodeExecutor::launchChained(
   if (error.empty()) error = stepSequence(bucket, false, sequence);
   if (error.empty()) error = sequence->launch();
   if (error.empty() && registry_) registry_->completed(bucket.uses);
-  if (error.empty() &&
-      tmc_decode_chain(static_cast<const std::int32_t*>(nextTokens_->devicePointer()),
-                       static_cast<std::int32_t*>(tokensView_->devicePointer()),
-                       static_cast<std::int32_t*>(lengthsView_->devicePointer()),
-                       static_cast<std::int32_t*>(history_->devicePointer()) + historyStep * M,
-                       static_cast<std::int64_t>(rows), runtime_->stream()) != 0)
+  if (error.empty() && runtime_->enqueue([&](void* stream) {
+        return tmc_decode_chain(
+            static_cast<const std::int32_t*>(nextTokens_->devicePointer()),
+            static_cast<std::int32_t*>(tokensView_->devicePointer()),
+            static_cast<std::int32_t*>(lengthsView_->devicePointer()),
+            static_cast<std::int32_t*>(history_->devicePointer()) + historyStep * M,
+            static_cast<std::int64_t>(rows), stream);
+      }) != 0)
     error = std::string("Chained decode: ") + tmc_last_error();
   std::fill(metaShadow_.begin(), metaShadow_.end(), std::numeric_limits<std::int32_t>::min());
   chainedRows_ = error.empty() ? rows : 0;

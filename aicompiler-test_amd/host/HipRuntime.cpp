@@ -412,6 +412,14 @@ SequencePreparationResult HipRuntime::prepareSequence(
 
 void* HipRuntime::stream() const noexcept { return runtime_ ? tmc_rt_stream(runtime_) : nullptr; }
 
+int HipRuntime::enqueue(const std::function<int(void*)>& work) const {
+  return tmc_rt_enqueue(
+      runtime_, [](void* stream, void* arg) {
+        return (*static_cast<const std::function<int(void*)>*>(arg))(stream);
+      },
+      const_cast<std::function<int(void*)>*>(&work));
+}
+
 std::string HipRuntime::synchronize() const {
   if (!isAvailable()) return initializationError();
   return tmc_rt_synchronize(runtime_) == 0 ? std::string() : lastError("Synchronize failed.");
@@ -420,9 +428,11 @@ std::string HipRuntime::synchronize() const {
 std::string HipRuntime::fillNormal(const BufferHandle& buffer, std::uint64_t seed, float mean,
                                    float stddev) const {
   if (!buffer) return "Cannot fill a missing buffer.";
-  if (tmc_fill_normal(buffer->devicePointer(), static_cast<int>(buffer->elementType()),
-                      static_cast<int64_t>(buffer->elementCount()), seed, mean, stddev,
-                      stream()) != 0)
+  if (enqueue([&](void* stream) {
+        return tmc_fill_normal(buffer->devicePointer(), static_cast<int>(buffer->elementType()),
+                               static_cast<int64_t>(buffer->elementCount()), seed, mean, stddev,
+                               stream);
+      }) != 0)
     return lastError("Fill failed.");
   return {};
 }

@@ -17,6 +17,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <optional>
 #include <string>
@@ -248,9 +249,11 @@ class HipRuntime {
   [[nodiscard]] SequencePreparationResult prepareSequence(
       const std::vector<const PreparedExecution*>& steps) const;
 
-  // gfx950 additions: the stream every execution uses, a wait on it, a
+  // gfx950 additions: the stream every execution uses, work queued on it in
+  // turn with other threads' calls (tmc_rt_enqueue), a wait on it, a
   // device-side normal fill (synthetic weights) and the failure-injection hook.
   [[nodiscard]] void* stream() const noexcept;
+  [[nodiscard]] int enqueue(const std::function<int(void*)>& work) const;
   [[nodiscard]] std::string synchronize() const;
   [[nodiscard]] std::string fillNormal(const BufferHandle& buffer, std::uint64_t seed,
                                        float mean, float stddev) const;

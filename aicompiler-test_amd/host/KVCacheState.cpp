@@ -302,9 +302,11 @@ std::string KVCacheState::spillPages(hip::HipRuntime& runtime, KVPageSpill& out)
   auto* pagesBase = static_cast<unsigned char*>(raw) + header;
   const auto count = static_cast<std::int64_t>(out.pages);
   const auto bytes = static_cast<std::int64_t>(out.pageBytes);
-  if (tmc_copy_pages(key_->devicePointer(), pagesBase, ids, count, bytes, 0, runtime.stream()) != 0 ||
-      tmc_copy_pages(value_->devicePointer(), pagesBase + out.pages * out.pageBytes, ids, count,
-                     bytes, 0, runtime.stream()) != 0)
+  if (runtime.enqueue([&](void* stream) {
+        return tmc_copy_pages(key_->devicePointer(), pagesBase, ids, count, bytes, 0, stream) != 0 ||
+               tmc_copy_pages(value_->devicePointer(), pagesBase + out.pages * out.pageBytes, ids,
+                              count, bytes, 0, stream) != 0;
+      }) != 0)
     return tmc_last_error();
   return runtime.synchronize();
 }
@@ -326,9 +328,11 @@ std::string KVCacheState::restorePages(hip::HipRuntime& runtime, const KVPageSpi
   const auto* pagesBase = static_cast<const unsigned char*>(spill.host.get()) + header;
   const auto count = static_cast<std::int64_t>(spill.pages);
   const auto bytes = static_cast<std::int64_t>(pageBytes);
-  if (tmc_copy_pages(pagesBase, key_->devicePointer(), ids, count, bytes, 1, runtime.stream()) != 0 ||
-      tmc_copy_pages(pagesBase + spill.pages * pageBytes, value_->devicePointer(), ids, count, bytes,
-                     1, runtime.stream()) != 0)
+  if (runtime.enqueue([&](void* stream) {
+        return tmc_copy_pages(pagesBase, key_->devicePointer(), ids, count, bytes, 1, stream) != 0 ||
+               tmc_copy_pages(pagesBase + spill.pages * pageBytes, value_->devicePointer(), ids,
+                              count, bytes, 1, stream) != 0;
+      }) != 0)
     error = tmc_last_error();
   if (error.empty()) error = runtime.synchronize();
   if (!error.empty()) {

@@ -73,8 +73,17 @@ int tmc_rt_is_available(const tmc_runtime *rt);
 const char *tmc_rt_device_name(const tmc_runtime *rt);
 const char *tmc_rt_init_error(const tmc_runtime *rt);
 int tmc_rt_device_info(const tmc_runtime *rt, tmc_hardware_info *info);
-/* The stream every prepared execution and sequence of this runtime uses. */
+/* The stream every prepared execution and sequence of this runtime uses.
+ * Calls on the runtime take turns queuing their work; what a thread queues on
+ * this handle itself may fall between the kernels of another thread's
+ * sequence, replayed as a graph or not (tmc_rt_enqueue takes its turn). */
 void *tmc_rt_stream(const tmc_runtime *rt);
+/* Calls work(stream, arg), which queues work on that stream and returns 0 or
+ * an error, where no other thread's call on this runtime can queue anything
+ * in between; returns its result.  `work` must not call a function that takes
+ * the runtime or an object of it.  No counterpart in the reference, whose
+ * command buffers are committed whole. */
+int tmc_rt_enqueue(tmc_runtime *rt, int (*work)(void *stream, void *arg), void *arg);
 /* Wait for all work enqueued on that stream (the reference's execute() is
  * synchronous; this is the wait for work enqueued with tmc_seq_launch). */
 int tmc_rt_synchronize(tmc_runtime *rt);
@@ -168,8 +177,9 @@ void tmc_exec_release(tmc_exec *exec);
  * six nodes (their launches cost less than the graph's), queues its steps'
  * launches in order on the runtime's stream instead; the small graph is still
  * what is launched while that stream is being captured.  Either way the steps
- * and their buffers must outlive the sequence, and what other threads queue on
- * the runtime falls before or after the whole replay. */
+ * and their buffers must outlive the sequence, and what other threads' calls
+ * on the runtime queue falls before or after the whole replay (not so what
+ * they queue on its stream's handle themselves, see tmc_rt_stream). */
 int tmc_seq_create(tmc_runtime *rt, tmc_exec *const *steps, size_t n, tmc_seq **out);
 int tmc_seq_run(tmc_seq *seq, double *gpu_us, double *cpu_us);
 /* Enqueue one replay on the runtime stream without waiting. */

@@ -37,32 +37,68 @@ def test_sequences_of_two_threads_do_not_interleave(tmc):
     one runtime: each output comes from its own input."""
     import torch
     rt = tmc.Runtime()
-    n = 1 << 16
+    n, replays = 1 << 14, 200
     make = lambda v: torch.full((n,), v, dtype=torch.float32, device="cuda")  # noqa: E731
-    a, b, scratch, oa, ob = make(1.0), make(100.0), make(0.0), make(0.0), make(0.0)
     key = rt.resolve(f"add?count={n}&dtype=f32")
-    wrap = {id(t): rt.wrap(t) for t in (a, b, scratch, oa, ob)}
-    zero = rt.wrap(make(0.0))
-    w = lambda t: wrap[id(t)]  # noqa: E731
+    zero, scratch = rt.wrap(make(0.0)), rt.wrap(make(0.0))
+    # every replay has an output of its own, so a wrong one stays to be seen
+    outs = torch.zeros((2, replays, n), dtype=torch.float32, device="cuda")
     seqs = []
-    for src, dst in ((a, oa), (b, ob)):
-        seqs.append(rt.sequence([rt.prepare(key, [w(src), zero], [w(scratch)]),
-                                 rt.prepare(key, [w(scratch), zero], [w(dst)])]))
+    for i, value in enumerate((1.0, 100.0)):
+        first = rt.prepare(key, [rt.wrap(make(value)), zero], [scratch])
+        seqs.append([rt.sequence([first, rt.prepare(key, [scratch, zero], [rt.wrap(o)])])
+                     for o in outs[i]])
     torch.cuda.synchronize()
-    bad = []
+    start = threading.Barrier(2)
 
     def work(i):
-        for _ in range(300):
-            seqs[i].launch()
+        start.wait()
+        for seq in seqs[i]:
+            seq.launch()
 
-    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    _run_threads([lambda i=i: work(i) for i in range(2)])
+    torch.cuda.synchronize()
+    assert bool((outs[0] == 1.0).all()), "the second thread's scratch reached the first's outputs"
+    assert bool((outs[1] == 100.0).all()), "the first thread's scratch reached the second's outputs"
+
+
+def _two_writes(tmc, rt, torch, pairs, n=1 << 14):
+    """A sequence of `pairs` times a kernel that stores 2 and one that stores
+    100 into one buffer, which holds 100 before and after a replay."""
+    make = lambda v: torch.full((n,), v, dtype=torch.float32, device="cuda")  # noqa: E731
+    key = rt.resolve(f"add?count={n}&dtype=f32")
+    zero, out = rt.wrap(make(0.0)), make(100.0)
+    buf = rt.wrap(out)
+    steps = [rt.prepare(key, [rt.wrap(make(v)), zero], [buf]) for v in (2.0, 100.0)]
+    torch.cuda.synchronize()
+    return buf, rt.sequence(steps * pairs)
+
+
+def _run_threads(bodies):
+    threads = [threading.Thread(target=b) for b in bodies]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
+
+
+@pytest.mark.parametrize("pairs", [1, 3, 5])
+def test_a_read_sees_whole_replays(tmc, pairs):
+    """A buffer read from another thread falls before or after a replay."""
+    import torch
+    rt = tmc.Runtime()
+    buf, seq = _two_writes(tmc, rt, torch, pairs)
+    done, seen = threading.Event(), set()
+
+    def launch():
+        for _ in range(3000):
+            seq.launch()
+        done.set()
+
+    def read():
+        while not done.is_set():
+            seen.update(set(buf.read_raw().tolist()))
+
+    _run_threads([launch, read])
     torch.cuda.synchronize()
-    if not bool((oa == 1.0).all()):
-        bad.append("first")
-    if not bool((ob == 100.0).all()):
-        bad.append("second")
-    assert not bad
+    assert seen == {100.0}, seen
