@@ -735,7 +735,9 @@ __device__ __forceinline__ void consume_step(const AttnParams& p, const int* s_p
 // 16db + n of positions 16h + 4g .. +3.  The probabilities are the A operand
 // just as the score MFMA left them: lane (head j, group g) holds positions
 // 4g .. 4g+3 of both 16-position tiles, the same k order.  oacc[db][r] is
-// O[head 4g + r][16 db + j], summed over the positions of the steps so far.
+// O[head 4g + r][16 db + j], summed over the positions of the steps so far
+// (D = 64: times kRaise).
+constexpr float kRaise = 32768.0f;
 template <int D, int GROUP, int MODE>
 __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvStep<D, MODE>& st,
                                                  const h8 (&qb)[D / 32], int p0, int end, int j,
@@ -792,8 +794,11 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
   const float next = fmaxf(m, tile_max);
   const float alpha = next == -INFINITY ? 1.0f : fast_exp2(m - next);
   float psum = 0.0f;
-  // D = 64: fp16 weights and what their rounding left, so that the product
-  // keeps the fp32 weights of the VALU form (21 bits of them)
+  // D = 64: fp16 weights and what their rounding left, in place of the fp32
+  // weights of the VALU form.  They are raised by kRaise (taken off the output
+  // again), so that 22 bits are left of every weight above 2^-18 of the
+  // greatest and an error of 2^-40 of it below; unraised, the second part ended
+  // at 2^-25, and weights of 2^-16 kept 9 bits.
   constexpr bool kSplitP = D != 128;
   h8 pa, pl;
 #pragma unroll
@@ -802,7 +807,7 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
     for (int r = 0; r < 4; ++r) {
       const float pr = sc[t][r] == -INFINITY ? 0.0f : fast_exp2(sc[t][r] - next);
       psum += pr;
-      const float pw = j < GROUP ? pr : 0.0f;
+      const float pw = j < GROUP ? (kSplitP ? pr * kRaise : pr) : 0.0f;
       pa[4 * t + r] = (half_t)pw;
       if constexpr (kSplitP) pl[4 * t + r] = (half_t)(pw - (float)pa[4 * t + r]);
     }
@@ -1067,7 +1072,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
     for (int r = 0; r < 4; ++r)
       if (4 * g + r < GROUP)
 #pragma unroll
-        for (int db = 0; db < D / 16; ++db) s_o[wave][4 * g + r][16 * db + j] = oacc[db][r];
+        for (int db = 0; db < D / 16; ++db)
+          s_o[wave][4 * g + r][16 * db + j] = D != 128 ? oacc[db][r] / kRaise : oacc[db][r];
   } else {
 #pragma unroll
     for (int h = 0; h < GROUP; ++h)

@@ -89,3 +89,33 @@ def test_contiguous_d64_matches_fp64(tmc, b, qh, kvh, capacity, length):
                    v[i, :, :length].transpose(0, 1))
         err = (out[i].view(qh, d).double() - ref).abs().max().item()
         assert err <= TOL, (i, err)
+
+
+@pytest.mark.parametrize("qh,kvh,gap,length", [(8, 2, 12.5, 500), (8, 1, 16.4, 2000),
+                                               (32, 8, 20.6, 1000), (8, 2, 22.4, 4000)])
+def test_small_weights_keep_their_bits(tmc, qh, kvh, gap, length):
+    """One position holds the greatest weight and a value of zero, all others
+    weigh 2^-gap of it: the output is theirs alone.  fp32 weights (or two fp16
+    parts of 22 bits in all, down to 2^-18, and 2^-40 absolute below) leave its
+    own fp16 rounding, 2^-11, and up to 2^-40 / 2^-gap of it."""
+    import torch
+    torch.manual_seed(gap)
+    d, p = 64, 16
+    capacity = -(-length // p) * p
+    pages = capacity // p
+    k = torch.zeros((pages, kvh, p, d), dtype=torch.float16, device="cuda")
+    v = (torch.rand((pages, kvh, p, d), device="cuda") + 1).half() * 2 ** int(gap - 10)
+    v[length // 3 // p, :, length // 3 % p] = 0
+    k[length // 3 // p, :, length // 3 % p, 0] = gap * math.log(2)
+    q = torch.zeros((1, qh, d), dtype=torch.float16, device="cuda")
+    q[..., 0] = 8
+    i32 = lambda x: torch.as_tensor(x, dtype=torch.int32).cuda()  # noqa: E731
+    out = torch.full((1, qh * d), float("nan"), dtype=torch.float16, device="cuda")
+    ws = torch.zeros(max(tmc.attention_workspace_bytes(1, qh, kvh, d, capacity) // 4, 1),
+                     dtype=torch.float32, device="cuda")
+    tmc.paged_decode_attention(q.view(1, -1), k, v, i32([length]), i32(list(range(pages))), i32([1]),
+                               out, 1, qh, kvh, d, p, pages, kvh * p * d, p * d, ws)
+    flat = [t.permute(0, 2, 1, 3).reshape(-1, kvh, d)[:length] for t in (k, v)]
+    ref = _ref(torch, q[0], *flat)
+    err = ((out[0].view(qh, d).double() - ref).abs() / ref.abs()).max().item()
+    assert err <= 2 ** -11 + 2 ** -20 + 2.0 ** (gap - 38), err
