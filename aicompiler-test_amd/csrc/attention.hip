@@ -797,7 +797,7 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
   // D = 64: fp16 weights and what their rounding left, in place of the fp32
   // weights of the VALU form.  They are raised by kRaise (taken off the output
   // again), so that 22 bits are left of every weight above 2^-18 of the
-  // greatest and an error of 2^-40 of it below; unraised, the second part ended
+  // greatest and an error of 2^-37 of it below; unraised, the second part ended
   // at 2^-25, and weights of 2^-16 kept 9 bits.
   constexpr bool kSplitP = D != 128;
   h8 pa, pl;
@@ -807,10 +807,36 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
     for (int r = 0; r < 4; ++r) {
       const float pr = sc[t][r] == -INFINITY ? 0.0f : fast_exp2(sc[t][r] - next);
       psum += pr;
-      const float pw = j < GROUP ? (kSplitP ? pr * kRaise : pr) : 0.0f;
-      pa[4 * t + r] = (half_t)pw;
-      if constexpr (kSplitP) pl[4 * t + r] = (half_t)(pw - (float)pa[4 * t + r]);
+      if constexpr (kSplitP)
+        sc[t][r] = pr * kRaise;
+      else
+        pa[4 * t + r] = (half_t)(j < GROUP ? pr : 0.0f);
     }
+  if constexpr (kSplitP) {
+    // Both parts of a positive weight are positive (the first is cut, not
+    // rounded, and neither is below 2^-24), so an infinite V meets no zero and
+    // no opposite sign: the output is that infinity, as with one weight.  The
+    // shift by at most 2^-22 is 2^-37 of the greatest weight.  (Lanes past the
+    // group hold weights of rows that are not stored.)
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      float whole[2], least[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float pw = sc[(e + h) / 4][(e + h) % 4];
+        least[h] = pw > 0.0f ? 0x1p-24f : 0.0f;
+        whole[h] = fmaxf(pw, 2.0f * least[h]);
+      }
+      typedef half_t v2h __attribute__((ext_vector_type(2)));
+      const v2h top =
+          __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(whole[0], whole[1]));
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        pa[e + h] = top[h];
+        pl[e + h] = (half_t)(whole[h] - (float)top[h] + least[h]);
+      }
+    }
+  }
   lsum = lsum * alpha + psum;
   m = next;
   // rows 4g .. 4g+3 of the accumulator are heads 4g + r: their alpha

@@ -96,8 +96,8 @@ def test_contiguous_d64_matches_fp64(tmc, b, qh, kvh, capacity, length):
 def test_small_weights_keep_their_bits(tmc, qh, kvh, gap, length):
     """One position holds the greatest weight and a value of zero, all others
     weigh 2^-gap of it: the output is theirs alone.  fp32 weights (or two fp16
-    parts of 22 bits in all, down to 2^-18, and 2^-40 absolute below) leave its
-    own fp16 rounding, 2^-11, and up to 2^-40 / 2^-gap of it."""
+    parts of 22 bits in all down to 2^-18, and 2^-37 absolute below) leave its
+    own fp16 rounding, 2^-11, and up to 2^-37 / 2^-gap of it."""
     import torch
     torch.manual_seed(gap)
     d, p = 64, 16
@@ -119,3 +119,44 @@ def test_small_weights_keep_their_bits(tmc, qh, kvh, gap, length):
     ref = _ref(torch, q[0], *flat)
     err = ((out[0].view(qh, d).double() - ref).abs() / ref.abs()).max().item()
     assert err <= 2 ** -11 + 2 ** -20 + 2.0 ** (gap - 38), err
+
+
+@pytest.mark.parametrize("qh,kvh,p,length,capacity", [(8, 2, 16, 300, 512), (8, 1, 16, 700, 4096),
+                                                      (8, 2, 12, 300, 516), (8, 8, 16, 300, 512)])
+def test_infinite_values_stay_infinite(tmc, qh, kvh, p, length, capacity):
+    """A V element of +-inf makes its column +-inf, two of opposite sign NaN,
+    and reaches nothing else: GQA on the MFMA kernel as on the VALU one (page
+    size 12) and in the one-block rows."""
+    import torch
+    torch.manual_seed(p + length)
+    d, pages = 64, -(-capacity // p)
+    k, v = (torch.randn((pages, kvh, p, d), device="cuda").half() for _ in range(2))
+    q = torch.randn((1, qh * d), device="cuda").half()
+    flat = v.permute(0, 2, 1, 3).reshape(-1, kvh, d).clone()
+    inf = float("inf")
+    put = lambda at, head, col, x: v[at // p, head, at % p].__setitem__(col, x)  # noqa: E731
+    for at in range(0, length, 7):
+        put(at, 0, 3, inf)
+    put(length - 1, 0, 10, inf)
+    put(31, kvh - 1, 20, -inf)
+    put(5, 0, 40, inf)
+    put(length // 2, 0, 40, -inf)
+    put(length, 0, 50, inf)  # past the row's length
+    i32 = lambda x: torch.as_tensor(x, dtype=torch.int32).cuda()  # noqa: E731
+    out = torch.zeros((1, qh * d), dtype=torch.float16, device="cuda")
+    ws = torch.zeros(max(tmc.attention_workspace_bytes(1, qh, kvh, d, pages * p) // 4, 1),
+                     dtype=torch.float32, device="cuda")
+    tmc.paged_decode_attention(q, k, v, i32([length]), i32(list(range(pages))), i32([1]), out, 1,
+                               qh, kvh, d, p, pages, kvh * p * d, p * d, ws)
+    kf = k.permute(0, 2, 1, 3).reshape(-1, kvh, d)[:length]
+    want = _ref(torch, q.view(qh, d), kf, flat[:length])
+    g = qh // kvh
+    want[:g, 3] = want[:g, 10] = inf
+    want[qh - g:, 20] = -inf
+    want[:g, 40] = float("nan")
+    got = out.view(qh, d).double()
+    assert bool((torch.isnan(got) == torch.isnan(want)).all())
+    for sign in (inf, -inf):
+        assert bool(((got == sign) == (want == sign)).all())
+    fin = torch.isfinite(want)
+    assert (got - want)[fin].abs().max().item() <= TOL
