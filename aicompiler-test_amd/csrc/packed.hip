@@ -375,16 +375,15 @@ int64_t packed_elements(int64_t n, int64_t k) { return ((n + 15) / 16) * 16 * ((
 // tile; narrow N needs more waves per tile to fill 256 CUs.  (Sharing each
 // activation fragment across 2 or 4 output tiles per block measured slower
 // at batch 16: the activation loads do not bound these kernels.)
-void default_packed(int64_t batch, int64_t n, int mats, int& unroll, int& ks) {
-  unroll = 2;
-  if (mats == 2)
-    ks = 4;
-  else if (n >= 16384)
-    ks = 1;
-  else if (n >= 8192)
-    ks = batch > 8 ? 2 : 4;
-  else
-    ks = batch >= 8 ? 16 : 8;
+struct PackedForm {
+  int unroll, ks;
+  bool chosen;  // by the caller: every pass runs this unroll and k split
+};
+PackedForm default_packed(int64_t batch, int64_t n, int mats) {
+  if (mats == 2) return {2, 4, false};
+  if (n >= 16384) return {2, 1, false};
+  if (n >= 8192) return {2, batch > 8 ? 2 : 4, false};
+  return {2, batch >= 8 ? 16 : 8, false};
 }
 
 // K tiles in flight per wave of the norm-folded LM head (N >= 16384, one
@@ -401,9 +400,12 @@ int lm_head_unroll(int64_t batch) { return batch > 8 ? 1 : 4; }
 // What bounds a launch from there is not HBM but the activation fragments,
 // which every output tile re-reads from L2 (about 15 TB/s over the chip).
 // The two-matrix form holds at most 8 waves' partial sums in 64 KiB of LDS.
-int row_tiles(int64_t batch, int64_t k, int mats, int ks) {
-  const int64_t mt = std::min<int64_t>(4, (batch + 15) / 16);
-  const bool fits = (uint64_t)64 * ((k + 31) / 32 * 32) * 2 < kNone && (mats == 1 || ks <= 8);
+// A caller's unroll bounds the tiles whose loads it holds in registers: four
+// row tiles at 1, two at 2, one at 4.
+int row_tiles(int64_t batch, int64_t k, int mats, const PackedForm& form) {
+  const int64_t most = form.chosen ? 4 / form.unroll : 4;
+  const int64_t mt = std::min(most, (batch + 15) / 16);
+  const bool fits = (uint64_t)64 * ((k + 31) / 32 * 32) * 2 < kNone && (mats == 1 || form.ks <= 8);
   return fits ? (int)mt : 1;
 }
 
@@ -427,19 +429,19 @@ int column_tiles(int mt, int64_t n, int mats) {
 template <int MATS, typename OutT, bool XP, bool YP, bool ROPE = false, int FUSE = kPackedPlain,
           bool ARGMAX = false>
 int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int64_t batch,
-               int64_t k, int64_t n, int unroll, int ks, hipStream_t st,
+               int64_t k, int64_t n, const PackedForm& form, hipStream_t st,
                const RopeArgs& rope = RopeArgs{}, const PackedFuseArgs& fuse = PackedFuseArgs{}) {
   const int64_t bytes = packed_elements(n, k) * 2;
   const int64_t x_pass = XP ? ((k + 31) / 32) * 512 : 16 * k;  // elements per 16-row pass
   const int64_t y_pass = YP ? ((n + 31) / 32) * 512 : 16 * n;
-  const int tiles = row_tiles(batch, k, MATS, ks);
+  const int tiles = row_tiles(batch, k, MATS, form);
   for (int64_t r0 = 0; r0 < batch; r0 += 16 * tiles) {
     const int rows = (int)std::min<int64_t>(16 * tiles, batch - r0);
     const int mt = (rows + 15) / 16;
-    const int nt = FUSE == kPackedResidual ? 1 : column_tiles(mt, n, MATS);
+    const int nt = FUSE == kPackedResidual || form.chosen ? 1 : column_tiles(mt, n, MATS);
     // of this pass alone: the last one may hold fewer row tiles, and then one
     // column tile, whose norm form is built for kPackedNormWaves waves
-    const int waves = nt > 1 ? 8 : ks;
+    const int waves = nt > 1 ? 8 : form.ks;
     TMC_REQUIRE(waves * kWave <= packed_threads(MATS, nt, mt, FUSE),
                 "Packed GEMM: internal error (more waves than the kernel's bound).");
     const dim3 grid((unsigned)(((n + 15) / 16 + nt - 1) / nt));
@@ -463,9 +465,10 @@ int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int
       }
     } else if (mt == 4) TMC_PACKED_LAUNCH(1, 4, 1);
     else if (mt == 3) TMC_PACKED_LAUNCH(1, 3, 1);
+    else if (mt == 2 && form.chosen && form.unroll == 1) TMC_PACKED_LAUNCH(1, 2, 1);
     else if (mt == 2) TMC_PACKED_LAUNCH(1, 2, 2);
-    else if (unroll == 1) TMC_PACKED_LAUNCH(1, 1, 1);
-    else if (unroll == 2) TMC_PACKED_LAUNCH(1, 1, 2);
+    else if (form.unroll == 1) TMC_PACKED_LAUNCH(1, 1, 1);
+    else if (form.unroll == 2) TMC_PACKED_LAUNCH(1, 1, 2);
     else TMC_PACKED_LAUNCH(1, 1, 4);
 #undef TMC_PACKED_LAUNCH
     if (check_launch("packed_gemm_kernel")) return 1;
@@ -475,21 +478,21 @@ int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int
 
 template <int MATS, typename OutT, int FUSE = kPackedPlain>
 int run_packed_layout(const half_t* x, const half_t* p0, const half_t* p1, OutT* y,
-                      int64_t batch, int64_t k, int64_t n, int unroll, int ks, int layout,
+                      int64_t batch, int64_t k, int64_t n, const PackedForm& form, int layout,
                       hipStream_t st, const PackedFuseArgs& pf = PackedFuseArgs{}) {
   const bool xp = layout & TMC_LAYOUT_X_PACKED, yp = layout & TMC_LAYOUT_Y_PACKED;
   const RopeArgs none{};
   if (xp && yp)
-    return run_packed<MATS, OutT, true, true, false, FUSE>(x, p0, p1, y, batch, k, n, unroll, ks,
-                                                           st, none, pf);
+    return run_packed<MATS, OutT, true, true, false, FUSE>(x, p0, p1, y, batch, k, n, form, st,
+                                                            none, pf);
   if (xp)
-    return run_packed<MATS, OutT, true, false, false, FUSE>(x, p0, p1, y, batch, k, n, unroll, ks,
-                                                            st, none, pf);
+    return run_packed<MATS, OutT, true, false, false, FUSE>(x, p0, p1, y, batch, k, n, form, st,
+                                                            none, pf);
   if (yp)
-    return run_packed<MATS, OutT, false, true, false, FUSE>(x, p0, p1, y, batch, k, n, unroll, ks,
-                                                            st, none, pf);
-  return run_packed<MATS, OutT, false, false, false, FUSE>(x, p0, p1, y, batch, k, n, unroll, ks,
-                                                           st, none, pf);
+    return run_packed<MATS, OutT, false, true, false, FUSE>(x, p0, p1, y, batch, k, n, form, st,
+                                                            none, pf);
+  return run_packed<MATS, OutT, false, false, false, FUSE>(x, p0, p1, y, batch, k, n, form, st,
+                                                            none, pf);
 }
 
 // One thread per 8-element slot of a 16-row pass in fragment order.
@@ -531,18 +534,15 @@ int packed_entry(int mats, const void* x, const void* p0, const void* p1, void* 
   TMC_REQUIRE((uint64_t)packed_elements(n, k) * 2 < kNone && (uint64_t)16 * k * 2 < kNone &&
                   n < (1LL << 31) && batch < (1LL << 31),
               std::string(what) + ": operands exceed the 4 GiB buffer range.");
-  int unroll, ks;
-  default_packed(batch, n, mats, unroll, ks);
+  PackedForm form = default_packed(batch, n, mats);
   // folded norm: 4 waves per tile below the LM head's width (batch 16 q.k.v
   // 20.5-20.9 us against 21.5 with the plain default of 2)
-  if (fuse == kPackedNorm) ks = n >= 16384 ? std::min(ks, kPackedNormWaves) : kPackedNormWaves;
-  if (fuse == kPackedNorm && n >= 16384) unroll = lm_head_unroll(batch);
-  if (config && config->algorithm != 0) {
-    unroll = config->unroll;
-    ks = config->k_split;
-  }
-  TMC_REQUIRE((unroll == 1 || unroll == 2 || unroll == 4) && ks >= 1 &&
-                  ks <= (fuse == kPackedNorm ? kPackedNormWaves : 16),
+  if (fuse == kPackedNorm)
+    form.ks = n >= 16384 ? std::min(form.ks, kPackedNormWaves) : kPackedNormWaves;
+  if (fuse == kPackedNorm && n >= 16384) form.unroll = lm_head_unroll(batch);
+  if (config && config->algorithm != 0) form = {config->unroll, config->k_split, true};
+  TMC_REQUIRE((form.unroll == 1 || form.unroll == 2 || form.unroll == 4) && form.ks >= 1 &&
+                  form.ks <= (fuse == kPackedNorm ? kPackedNormWaves : 16),
               std::string(what) + ": config needs unroll 1|2|4 and k_split 1..16 (1..4 with "
               "RMSNorm).");
   TMC_REQUIRE((layout & ~(TMC_LAYOUT_X_PACKED | TMC_LAYOUT_Y_PACKED)) == 0,
@@ -558,24 +558,24 @@ int packed_entry(int mats, const void* x, const void* p0, const void* p1, void* 
   if (fuse == kPackedNorm) {
     if (mats == 2)
       return run_packed_layout<2, half_t, kPackedNorm>(xs, a, b, static_cast<half_t*>(y), batch, k,
-                                                       n, unroll, ks, layout, st, pf);
+                                                       n, form, layout, st, pf);
     if (y_dtype == TMC_F32)
       return run_packed_layout<1, float, kPackedNorm>(xs, a, a, static_cast<float*>(y), batch, k,
-                                                      n, unroll, ks, layout & TMC_LAYOUT_X_PACKED,
+                                                      n, form, layout & TMC_LAYOUT_X_PACKED,
                                                       st, pf);
     return run_packed_layout<1, half_t, kPackedNorm>(xs, a, a, static_cast<half_t*>(y), batch, k,
-                                                     n, unroll, ks, layout, st, pf);
+                                                     n, form, layout, st, pf);
   }
   if (fuse == kPackedResidual)
     return run_packed_layout<1, half_t, kPackedResidual>(xs, a, a, static_cast<half_t*>(y), batch,
-                                                         k, n, unroll, ks, layout, st, pf);
+                                                         k, n, form, layout, st, pf);
   if (mats == 2)
-    return run_packed_layout<2, half_t>(xs, a, b, static_cast<half_t*>(y), batch, k, n, unroll,
-                                        ks, layout, st);
+    return run_packed_layout<2, half_t>(xs, a, b, static_cast<half_t*>(y), batch, k, n, form,
+                                        layout, st);
   if (y_dtype == TMC_F32)
-    return run_packed_layout<1, float>(xs, a, a, static_cast<float*>(y), batch, k, n, unroll, ks,
+    return run_packed_layout<1, float>(xs, a, a, static_cast<float*>(y), batch, k, n, form,
                                        layout & TMC_LAYOUT_X_PACKED, st);
-  return run_packed_layout<1, half_t>(xs, a, a, static_cast<half_t*>(y), batch, k, n, unroll, ks,
+  return run_packed_layout<1, half_t>(xs, a, a, static_cast<half_t*>(y), batch, k, n, form,
                                       layout, st);
 }
 
@@ -662,15 +662,11 @@ int qkv_rope_packed_entry(const void* x, bool norm, float eps, const void* packe
               "Packed q.k.v RoPE append: operands exceed the 4 GiB buffer range.");
   TMC_REQUIRE((layout & ~TMC_LAYOUT_X_PACKED) == 0,
               "Packed q.k.v RoPE append: layout may only set TMC_LAYOUT_X_PACKED.");
-  int unroll, ks;
-  default_packed(batch, n, 1, unroll, ks);
-  if (norm) ks = n >= 16384 ? std::min(ks, kPackedNormWaves) : kPackedNormWaves;
-  if (config && config->algorithm != 0) {
-    unroll = config->unroll;
-    ks = config->k_split;
-  }
-  TMC_REQUIRE((unroll == 1 || unroll == 2 || unroll == 4) && ks >= 1 &&
-                  ks <= (norm ? kPackedNormWaves : 16),
+  PackedForm form = default_packed(batch, n, 1);
+  if (norm) form.ks = n >= 16384 ? std::min(form.ks, kPackedNormWaves) : kPackedNormWaves;
+  if (config && config->algorithm != 0) form = {config->unroll, config->k_split, true};
+  TMC_REQUIRE((form.unroll == 1 || form.unroll == 2 || form.unroll == 4) && form.ks >= 1 &&
+                  form.ks <= (norm ? kPackedNormWaves : 16),
               "Packed q.k.v RoPE append: config needs unroll 1|2|4 and k_split 1..16 (1..4 with "
               "RMSNorm).");
   RopeArgs ra;
@@ -697,14 +693,14 @@ int qkv_rope_packed_entry(const void* x, bool norm, float eps, const void* packe
   if (norm) {
     if (layout & TMC_LAYOUT_X_PACKED)
       return run_packed<1, half_t, true, false, true, kPackedNorm>(xs, w, w, none, batch, hidden,
-                                                                   n, unroll, ks, st, ra, pf);
+                                                                   n, form, st, ra, pf);
     return run_packed<1, half_t, false, false, true, kPackedNorm>(xs, w, w, none, batch, hidden, n,
-                                                                  unroll, ks, st, ra, pf);
+                                                                  form, st, ra, pf);
   }
   if (layout & TMC_LAYOUT_X_PACKED)
-    return run_packed<1, half_t, true, false, true>(xs, w, w, none, batch, hidden, n, unroll, ks,
+    return run_packed<1, half_t, true, false, true>(xs, w, w, none, batch, hidden, n, form,
                                                     st, ra);
-  return run_packed<1, half_t, false, false, true>(xs, w, w, none, batch, hidden, n, unroll, ks, st,
+  return run_packed<1, half_t, false, false, true>(xs, w, w, none, batch, hidden, n, form, st,
                                                    ra);
 }
 
@@ -764,15 +760,12 @@ extern "C" int tmc_lm_head_partial_argmax_packed_norm_f16(
   TMC_REQUIRE((uint64_t)packed_elements(vocabulary, in_features) * 2 < kNone &&
                   (uint64_t)16 * in_features * 2 < kNone,
               what + ": operands exceed the 4 GiB buffer range.");
-  int unroll, ks;
-  default_packed(batch, vocabulary, 1, unroll, ks);
-  ks = vocabulary >= 16384 ? std::min(ks, kPackedNormWaves) : kPackedNormWaves;
-  if (vocabulary >= 16384) unroll = lm_head_unroll(batch);
-  if (config && config->algorithm != 0) {
-    unroll = config->unroll;
-    ks = config->k_split;
-  }
-  TMC_REQUIRE((unroll == 1 || unroll == 2 || unroll == 4) && ks >= 1 && ks <= kPackedNormWaves,
+  PackedForm form = default_packed(batch, vocabulary, 1);
+  form.ks = vocabulary >= 16384 ? std::min(form.ks, kPackedNormWaves) : kPackedNormWaves;
+  if (vocabulary >= 16384) form.unroll = lm_head_unroll(batch);
+  if (config && config->algorithm != 0) form = {config->unroll, config->k_split, true};
+  TMC_REQUIRE((form.unroll == 1 || form.unroll == 2 || form.unroll == 4) && form.ks >= 1 &&
+                  form.ks <= kPackedNormWaves,
               what + ": config needs unroll 1|2|4 and k_split 1..4.");
   PackedFuseArgs pf;
   pf.eps = epsilon;
@@ -783,9 +776,9 @@ extern "C" int tmc_lm_head_partial_argmax_packed_norm_f16(
   const RopeArgs none{};
   if (layout & TMC_LAYOUT_X_PACKED)
     return run_packed<1, float, true, false, false, kPackedNorm, true>(
-        xs, w, w, out, batch, in_features, vocabulary, unroll, ks, as_stream(stream), none, pf);
+        xs, w, w, out, batch, in_features, vocabulary, form, as_stream(stream), none, pf);
   return run_packed<1, float, false, false, false, kPackedNorm, true>(
-      xs, w, w, out, batch, in_features, vocabulary, unroll, ks, as_stream(stream), none, pf);
+      xs, w, w, out, batch, in_features, vocabulary, form, as_stream(stream), none, pf);
 }
 
 extern "C" int tmc_gate_up_silu_packed_norm_f16(const void* x, const void* packed_gate,

@@ -328,10 +328,11 @@ int tmc_pack_weights_scaled_f16(const void *w, const void *gamma, void *packed,
                                 int64_t out_features, int64_t in_features, void *stream);
 
 /* tmc_gemv_f16 / tmc_gate_up_silu_f16 semantics over packed weights, any
- * batch (16 rows per pass); in_features % 8 == 0, x and the packed buffers
- * 16-byte aligned.  config (may be NULL): algorithm 0 = default for the shape,
- * otherwise unroll 1|2|4 K tiles of 128 in flight and k_split 1..16 waves
- * per 16-row output tile. */
+ * batch (up to 64 rows per pass over the weights); in_features % 8 == 0, x
+ * and the packed buffers 16-byte aligned.  config (may be NULL): algorithm 0 =
+ * default for the shape, otherwise unroll 1|2|4 K tiles of 128 in flight (with
+ * up to 64, 32 or 16 rows per pass) and k_split 1..16 waves per 16-column
+ * output tile, in every pass. */
 int tmc_gemm_packed_f16(const void *x, const void *packed_w, void *y, int y_dtype, int64_t batch,
                         int64_t in_features, int64_t out_features, const tmc_gemv_config *config,
                         void *stream);

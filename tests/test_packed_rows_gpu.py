@@ -202,3 +202,47 @@ def test_norm_qkv_remainder_rows_equal_their_own_call(tmc, orc, torch, batch):
         out.extend(bits(t) for t in (q, kp, vp))
     for a, b in zip(whole, parts):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("unroll", [1, 2, 4])
+@pytest.mark.parametrize("batch,ks", [(24, 2), (40, 16), (64, 3), (70, 1)])
+def test_a_chosen_split_is_every_passes_split(tmc, orc, torch, batch, ks, unroll):
+    """A caller's k split and unroll hold above 16 rows and at widths whose
+    default is three column tiles: the bits of 16-row calls with them, with
+    the folded norm (at most 4 waves) as well."""
+    k, n = 1160, 12288
+    x = dev_f16(orc.f16(normal(2071 + batch, (batch, k))))
+    w = dev_f16(orc.f16(normal(2072, (n, k), 0.02)))
+    packed = tmc.pack_weights(w)
+
+    def rows(run, cfg):
+        return torch.cat([run(x[a:a + 16].contiguous(), cfg) for a in range(0, batch, 16)])
+
+    def plain(rows_x, cfg):
+        return _rows(tmc, torch, rows_x, packed, rows_x.shape[0], k, n, 1, cfg)
+
+    def norm(rows_x, cfg):
+        y = torch.full((rows_x.shape[0], n), float("nan"), dtype=torch.float32, device="cuda")
+        tmc.gemm_packed_norm(tmc.pack_activations(rows_x), packed, y, rows_x.shape[0], k, n, 1e-6, 1,
+                             cfg)
+        return y
+
+    cfg = tmc.GemvConfig(3, 1, unroll, ks)
+    assert torch.equal(plain(x, cfg), rows(plain, cfg))
+    cfg = tmc.GemvConfig(3, 1, unroll, min(ks, 4))
+    assert torch.equal(norm(x, cfg), rows(norm, cfg))
+
+
+@pytest.mark.parametrize("ks", [3, 16])
+def test_a_chosen_split_of_two_matrices(tmc, orc, torch, ks):
+    batch, k, n = 40, 1160, 11008
+    x = dev_f16(orc.f16(normal(2081, (batch, k))))
+    wg, wu = (tmc.pack_weights(dev_f16(orc.f16(normal(s, (n, k), 0.02)))) for s in (2082, 2083))
+    cfg = tmc.GemvConfig(3, 1, 1, ks)
+
+    def run(rows_x):
+        y = torch.full((rows_x.shape[0], n), float("nan"), dtype=torch.float16, device="cuda")
+        tmc.gate_up_silu_packed(rows_x, wg, wu, y, n, cfg)
+        return y
+
+    assert torch.equal(run(x), torch.cat([run(x[a:a + 16].contiguous()) for a in (0, 16, 32)]))
