@@ -72,7 +72,7 @@ struct PaBlockRegs {
 // position is at or past `end` or its page is absent).  BUF (pools below
 // 4 GiB): raw buffer loads with the out-of-range offset for absent data, so
 // every load issues unconditionally; otherwise predicated global loads.
-template <int D, bool BUF>
+template <int D, bool BUF, bool OFFS>
 __device__ __forceinline__ void pa_load(const PrefillParams& p, const int* table, int kvh, int base,
                                         int end, PaBlockRegs<D>& r) {
   using R = PaBlockRegs<D>;
@@ -82,6 +82,39 @@ __device__ __forceinline__ void pa_load(const PrefillParams& p, const int* table
   const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const __amdgpu_buffer_rsrc_t rk = buffer_resource(p.k, p.pool_bytes);
   const __amdgpu_buffer_rsrc_t rv = buffer_resource(p.v, p.pool_bytes);
+  if constexpr (OFFS) {
+    // `table` holds each page's byte offset for this kv head (kBufferAbsent
+    // for an absent page) and the page size is a power of two of at least 4:
+    // a 4-position V group lies in one page, so it costs one lookup.
+    const int shift = p.page_shift, mask = p.page_size - 1;
+    auto page_off = [&](int pos) -> unsigned {
+      return (unsigned)table[pos < end ? pos >> shift : 0];
+    };
+#pragma unroll
+    for (int i = 0; i < R::kPer; ++i) {
+      const int item = tid + i * kPaThreads;
+      const int pos = base + item / CH;
+      const unsigned off = page_off(pos);
+      const bool ok = pos < end && off != kBufferAbsent &&
+                      (R::kItems % kPaThreads == 0 || item < R::kItems);
+      r.k[i] = buffer_load_h8(
+          rk, ok ? off + (unsigned)(((pos & mask) * D + 8 * (item % CH)) * 2) : kBufferAbsent);
+    }
+#pragma unroll
+    for (int i = 0; i < R::vPer; ++i) {
+      const int item = tid + i * kPaThreads;
+      const int quad = item % (kPaBlock / 4), octet = item / (kPaBlock / 4);
+      const int pos0 = base + 4 * quad;
+      const unsigned off = page_off(pos0);
+      const unsigned row0 = off + (unsigned)(((pos0 & mask) * D + 8 * octet) * 2);
+      const bool group_ok = off != kBufferAbsent && (R::vItems % kPaThreads == 0 || item < R::vItems);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        r.v[q][i] = buffer_load_h8(
+            rv, group_ok && pos0 + q < end ? row0 + (unsigned)(q * D * 2) : kBufferAbsent);
+    }
+    return;
+  }
   const bool pow2 = p.page_shift >= 0;
   // Element offset of (pos, 8-element column), or -1 when absent; computed
   // with selects only (table[0] exists whenever end > 0).
@@ -224,8 +257,10 @@ __device__ __forceinline__ void pa_compute(const PrefillParams& p, const half_t*
 
 // TLDS: the request's block table is staged in LDS (dynamic, max_pages
 // entries) so a block's K/V addresses need no global round trip first.
-// BUF: see pa_load.  Serves what prefill_tile_kernel does not: pools of 4 GiB
-// and more, and block tables past kPtTable.
+// BUF: see pa_load.  With TLDS, BUF and a power-of-two page size of at
+// least 4 the LDS table holds byte offsets (pa_load's OFFS form).  Serves what
+// prefill_tile_kernel does not: strides that are no multiples of 8 halves,
+// block tables past kPtTable, and pools of 4 GiB and more.
 template <int D, bool TLDS, bool BUF>
 __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillParams p) {
   constexpr int KS = D / 32;  // k-steps of the score product
@@ -274,6 +309,7 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
     if (p.row_table && p.row_table[token] != tile_table) len = -1;
   }
 
+  const bool offs = TLDS && BUF && p.page_shift >= 2;  // workgroup-uniform
   // Attended extent of the tile and the first absent page below it.
   if (threadIdx.x == 0) {
     s_bounds[0] = 0;
@@ -290,7 +326,14 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
     for (int i = threadIdx.x; i < pages; i += kPaThreads) {
       const int page = request_table[i];
       const bool ok = page >= 0 && page < p.pool_pages;
-      if (TLDS) s_table[i] = page;
+      if (TLDS) {
+        if (offs)
+          s_table[i] = (int)(ok ? (unsigned)(((long)page * p.page_stride +
+                                              (long)kvh * p.head_stride) * 2)
+                                : kBufferAbsent);
+        else
+          s_table[i] = page;
+      }
       if (!ok) first_bad = min(first_bad, i);
     }
     if (first_bad != 0x7fffffff) atomicMin(&s_bounds[1], first_bad);
@@ -319,7 +362,10 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
   // and land during its compute.  (Two or three blocks in flight measured
   // no faster.)
   PaBlockRegs<D> regs;
-  auto load = [&](int at) { pa_load<D, BUF>(p, table, kvh, at, end, regs); };
+  auto load = [&](int at) {
+    if (offs) pa_load<D, BUF, TLDS && BUF>(p, table, kvh, at, end, regs);
+    else pa_load<D, BUF, false>(p, table, kvh, at, end, regs);
+  };
   load(0);
   for (int base = 0; base < end; base += kPaBlock) {
     __syncthreads();  // the previous block's LDS reads are done
@@ -760,7 +806,7 @@ extern "C" int tmc_prefill_attention_rows_f16(const void* q, const void* key_poo
   const size_t table_lds = (size_t)max_pages * 4;
   const bool tlds = static_lds + table_lds <= kPaMaxLds;
   const bool buf = (uint64_t)pool_pages * (uint64_t)page_stride * 2 < kBufferAbsent;
-  const size_t dyn = tlds && !buf ? table_lds : 0;
+  const size_t dyn = tlds ? table_lds : 0;
   const hipStream_t s = as_stream(stream);
   const uint64_t pool_bytes = (uint64_t)pool_pages * (uint64_t)page_stride * 2;
   p.pool_bytes = buf ? (unsigned)pool_bytes : 0u;
@@ -788,13 +834,17 @@ extern "C" int tmc_prefill_attention_rows_f16(const void* q, const void* key_poo
 #define TMC_PA_LAUNCH(DIM, T, B)                                                                  \
   hipLaunchKernelGGL((prefill_attention_kernel<DIM, T, B>), grid, dim3(kPaThreads), dyn, s, p)
   if (head_dim == 128) {
-    if (buf) TMC_PA_LAUNCH(128, false, true);
-    else if (tlds) TMC_PA_LAUNCH(128, true, false);
-    else TMC_PA_LAUNCH(128, false, false);
+    if (tlds) {
+      if (buf) TMC_PA_LAUNCH(128, true, true); else TMC_PA_LAUNCH(128, true, false);
+    } else {
+      if (buf) TMC_PA_LAUNCH(128, false, true); else TMC_PA_LAUNCH(128, false, false);
+    }
   } else {
-    if (buf) TMC_PA_LAUNCH(64, false, true);
-    else if (tlds) TMC_PA_LAUNCH(64, true, false);
-    else TMC_PA_LAUNCH(64, false, false);
+    if (tlds) {
+      if (buf) TMC_PA_LAUNCH(64, true, true); else TMC_PA_LAUNCH(64, true, false);
+    } else {
+      if (buf) TMC_PA_LAUNCH(64, false, true); else TMC_PA_LAUNCH(64, false, false);
+    }
   }
 #undef TMC_PA_LAUNCH
   return check_launch("prefill_attention_kernel");
