@@ -616,11 +616,15 @@ __device__ __forceinline__ h8 rsrc_h8(__amdgpu_buffer_rsrc_t r, unsigned byte_of
 //
 // A weight load reads 4 whole 256-byte rows of a tile (8 full cache lines)
 // and the tile is re-laid in the operand order through the wave's own LDS
-// slices (chunk c of row r at slot c ^ r); read in the operand order, a load
+// slices (chunk c of row r at slot c ^ r), two of them or, in blocks of more
+// than 8 waves, one, so that a block's slices stay within 64 KiB and two such
+// blocks fit a CU; read in the operand order, a load
 // touches 16 rows x 64 bytes, half lines of 16 DRAM rows.  MI355X, weights
 // beyond the caches: 8 x 4096 x 4096 9.3 -> 7.7 us, 8 x 4096 x 12288 26.9 ->
 // 19.6, gate/up 8 x 4096 x 11008 41.3 -> 31.6 (5.7 TB/s).  More tiles in
 // flight per wave (U) no longer help.
+constexpr int row_slices(int threads) { return threads > 8 * kWave ? 1 : 2; }
+
 template <int MATS, int RT, int MT, int U, int THREADS, typename OutT>
 __global__ __launch_bounds__(THREADS) void mfma_rows_kernel(
     const half_t* __restrict__ x, const half_t* __restrict__ w0, const half_t* __restrict__ w1,
@@ -654,7 +658,8 @@ __global__ __launch_bounds__(THREADS) void mfma_rows_kernel(
   const int per_wave = (tiles + ks_count - 1) / ks_count;
   const int first = ks * per_wave;
   const int last = min(tiles, first + per_wave);
-  h8* slices = reinterpret_cast<h8*>(red) + ks * 512;
+  constexpr int kSlices = row_slices(THREADS);
+  h8* slices = reinterpret_cast<h8*>(red) + ks * 256 * kSlices;
   for (int t0 = first; t0 < last; t0 += U) {
     h8 xv[U][MT][4], wv[U][MATS][RT][4];
 #pragma unroll
@@ -689,7 +694,7 @@ __global__ __launch_bounds__(THREADS) void mfma_rows_kernel(
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           h8 wf[4];
-          h8* slice = slices + 256 * ((u * MATS * RT + m * RT + rt) & 1);
+          h8* slice = slices + 256 * ((u * MATS * RT + m * RT + rt) % kSlices);
 #pragma unroll
           for (int s = 0; s < 4; ++s) slice[(4 * s + g) * 16 + (j ^ (4 * s + g))] = wv[u][m][rt][s];
           __builtin_amdgcn_wave_barrier();
@@ -920,7 +925,8 @@ int launch_rows(const Shape& s, const half_t* x, OutT* y, int rows, int ks, int 
                 hipStream_t st) {
   const dim3 grid((unsigned)((s.n + block_rows - 1) / block_rows));
   const size_t sums = (size_t)ks * MATS * RT * MT * 4 * kWave * sizeof(float);
-  const size_t lds = std::max(sums, (size_t)ks * 512 * sizeof(h8));  // or the waves' slices
+  const size_t slices = (size_t)ks * 256 * row_slices(THREADS) * sizeof(h8);
+  const size_t lds = std::max(sums, slices);  // the one after the other
   hipLaunchKernelGGL((mfma_rows_kernel<MATS, RT, MT, U, THREADS, OutT>), grid, dim3(ks * kWave), lds, st, x,
                      s.w0, s.w1, y, rows, s.n, s.k, ks, block_rows);
   return check_launch("mfma_rows_kernel");
@@ -928,7 +934,8 @@ int launch_rows(const Shape& s, const half_t* x, OutT* y, int rows, int ks, int 
 
 template <int MATS, typename OutT>
 int run_rows(const Shape& s, const tmc_gemv_config& cfg, hipStream_t st) {
-  // The LDS reduction holds k_split x MATS x tiles 16x16 fp32 partials.
+  // The LDS reduction holds k_split x MATS x tiles 16x16 fp32 partials; the
+  // waves' slices are within the same 64 KiB.
   TMC_REQUIRE((size_t)cfg.k_split * MATS * cfg.rows_per_wave * 4 * kWave * sizeof(float) <= 65536,
               "GEMV config: MFMA row tiles need k_split * tiles * matrices <= 64 (64 KiB LDS).");
   OutT* y = static_cast<OutT*>(s.y);

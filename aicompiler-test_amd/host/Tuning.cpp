@@ -115,7 +115,9 @@ std::size_t decodeGEMVLdsBytes(std::size_t batch, const DecodeGEMVConfig& c) {
     const std::size_t mt = std::min<std::size_t>(4, (std::min<std::size_t>(batch, 64) + 15) / 16);
     return static_cast<std::size_t>(c.rowsPerWave * c.kSplit) * (mt == 3 ? 4 : mt) * tile;
   }
-  case 3: return static_cast<std::size_t>(c.kSplit * c.rowsPerWave) * tile;
+  case 3:  // the partials, or the waves' weight slices before them
+    return static_cast<std::size_t>(c.kSplit) *
+           std::max<std::size_t>(c.rowsPerWave * tile, (c.kSplit > 8 ? 4 : 8) * 1024);
   case 4: return 0;
   case 5: return (4 * 35 * static_cast<std::size_t>(c.rowsPerWave) + 128) * sizeof(float);
   default: return 4 * static_cast<std::size_t>(c.rowsPerWave) * 8 * sizeof(float);

@@ -24,7 +24,8 @@ def test_row_major_linear_matches_fp64(tmc, orc, batch, k, n):
 
 
 @pytest.mark.parametrize("batch,k,n", [(2, 64, 9), (9, 4096, 11008), (30, 1160, 4097),
-                                       (50, 520, 3000), (64, 264, 33000)])
+                                       (50, 520, 3000), (64, 264, 33000), (40, 264, 9000),
+                                       (48, 520, 12288)])
 def test_row_major_gated_matches_fp64(tmc, orc, batch, k, n):
     import torch
     x = dev_f16(orc.f16(normal(4011 + batch, (batch, k))))

@@ -37,6 +37,9 @@ def test_decode_gemv_hardware_filter(host):
     assert "persistent" in ok(cfg(5, 1, 1, 4), batch=1, k=16392)
     assert ok(cfg(3, 4, 1, 16)) == ""                      # 64 KiB of partials: at the limit
     assert host.decode_gemv_lds_bytes(16, cfg(3, 4, 1, 16)) == 64 * 1024
+    # weight slices: 8 KiB a wave up to 8 waves, 4 KiB in larger blocks
+    assert host.decode_gemv_lds_bytes(16, cfg(3, 1, 1, 4)) == 32 * 1024
+    assert host.decode_gemv_lds_bytes(16, cfg(3, 1, 1, 16)) == 64 * 1024
     assert "LDS" in ok(cfg(3, 8, 1, 16))                   # 128 KiB at 1024 threads
     assert "64" in ok(cfg(2, 4, 1, 8))                     # 2048 threads
     assert "multiple of 8" in ok(cfg(1, 1, 2, 4), batch=1, k=4097)
