@@ -18,9 +18,10 @@
 //  * Linear baseline (algorithm 4): one thread per output, the reference
 //    tuner's baseline kept as the tuners' fallback.
 //
-//  * MFMA row-tile GEMM (algorithm 3, batch <= 16 per pass): the same
-//    instruction, but a wave owns RT 16-row output tiles (one activation
-//    fragment serves RT weight fragments) and every operand is read with raw
+//  * MFMA row-tile GEMM (algorithm 3, up to 64 batch rows per pass, 16 with a
+//    configuration of the caller's): the same instruction, but a wave owns RT
+//    16-row output tiles (one activation fragment serves RT weight fragments),
+//    weights are read in whole rows and every operand is read with raw
 //    buffer loads: rows past N, batch rows past B and k past K get an
 //    offset beyond the buffer, which reads as zero, so no load is
 //    predicated.  KS waves of a block split K; all waves share the LDS
@@ -1023,11 +1024,13 @@ int run_rows_default(const Shape& s, hipStream_t st) {
 // Default configuration per shape (the tuner may override it), from graph-
 // timed sweeps on MI355X with weights larger than the Infinity Cache: batch 1
 // streams rows with the dot algorithm and 4 waves per row (2 rows per wave
-// for rows longer than 8K); larger batches use the MFMA row-tile kernel.
-// Sweep winners (batch 8 / 16, K 4096 unless noted): N 12288 -> 1|2 tiles,
-// unroll 1, 4 waves; N 4096 (K 4096 and K 11008) -> 1 tile, 8 waves; N 32000
-// -> 2 tiles, unroll 1, 2 waves; gated N 11008 -> 1 tile, 4 waves, unroll 1
-// at batch 8 and 4 at batch 16.
+// for rows longer than 8K); larger batches use the MFMA row-tile kernel.  There
+// the configuration names the default, whose blocks run_rows_default shapes;
+// its values are those of the 16-row passes that serve batches whose 64 rows
+// of x are past 4 GiB (sweep winners at batch 8 / 16, K 4096 unless noted: N
+// 12288 1|2 tiles, unroll 1, 4 waves; N 4096, K 4096 and 11008, 1 tile, 8
+// waves; N 32000 2 tiles, unroll 1, 2 waves; gated N 11008 1 tile, 4 waves,
+// unroll 1 at batch 8 and 4 at batch 16).
 tmc_gemv_config default_config(int batch, int n, int k, int mats) {
   tmc_gemv_config c{};
   (void)k;
@@ -1072,6 +1075,11 @@ tmc_gemv_config default_config(int batch, int n, int k, int mats) {
     c.k_split = 8;
   }
   return c;
+}
+
+bool same_config(const tmc_gemv_config& a, const tmc_gemv_config& b) {
+  return a.algorithm == b.algorithm && a.rows_per_wave == b.rows_per_wave &&
+         a.unroll == b.unroll && a.k_split == b.k_split;
 }
 
 int validate_config(const tmc_gemv_config& c) {
@@ -1146,7 +1154,9 @@ int run_linear(int mats, const void* x, const void* w0, const void* w1, void* y,
     return check_launch("gemv_generic_kernel");
   }
   tmc_gemv_config cfg = default_config(s.batch, s.n, s.k, mats);
-  if (user && user->algorithm != 0) cfg = *user;
+  // the default's own configuration passed back names the default
+  const bool chosen = user && user->algorithm != 0 && !same_config(*user, cfg);
+  if (chosen) cfg = *user;
   if (validate_config(cfg)) return 1;
   if (cfg.algorithm == 5) {
     TMC_REQUIRE(s.batch == 1 && s.k <= 16384 &&
@@ -1170,7 +1180,6 @@ int run_linear(int mats, const void* x, const void* w0, const void* w1, void* y,
   if (cfg.algorithm == 3) {
     // raw buffers address at most 4 GiB - 16 bytes
     const uint64_t wb = (uint64_t)s.n * s.k * 2, xb = (uint64_t)min(s.batch, 64) * s.k * 2;
-    const bool chosen = user && user->algorithm != 0;
     if (wb < kNoData && xb < kNoData && !chosen) {
       if (mats == 2) return run_rows_default<2, half_t>(s, st);
       return y_dtype == TMC_F32 ? run_rows_default<1, float>(s, st)

@@ -210,7 +210,8 @@ int tmc_gemv_f16(const void *x, const void *w, void *y, int y_dtype, int64_t bat
  * <= 16, unroll 1|2 K tiles in flight), 3 = MFMA row tiles with buffer loads
  * (rows_per_wave 1|2|4 16-row tiles per wave, k_split 1..16 waves per block
  * each taking a contiguous K run, unroll 1|2|4 adjacent K tiles in flight,
- * 4 only with at most 2 tiles; batch handled 16 rows per pass), 4 = linear
+ * 4 only with at most 2 tiles; batch handled 16 rows per pass, up to 64 in
+ * the default's blocks), 4 = linear
  * baseline, one thread per output (emitLinearBaseline,
  * DecodeGEMVMetalEmitter.cpp:18-66; the tuners' baseline and fallback, other
  * fields ignored), 5 = persistent dot at batch 1 (no reference counterpart:
@@ -231,7 +232,8 @@ int tmc_gemv_f16_config(const void *x, const void *w, void *y, int y_dtype, int6
                         int64_t in_features, int64_t out_features, const tmc_gemv_config *config,
                         void *stream);
 
-/* The configuration tmc_gemv_f16 / tmc_gate_up_silu_f16 pick for a shape. */
+/* The configuration tmc_gemv_f16 / tmc_gate_up_silu_f16 pick for a shape.
+ * Passed to the _config forms it runs what they run, bit for bit. */
 int tmc_gemv_default_config(int64_t batch, int64_t in_features, int64_t out_features, int gated,
                             tmc_gemv_config *out);
 

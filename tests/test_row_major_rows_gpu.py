@@ -38,6 +38,30 @@ def test_row_major_gated_matches_fp64(tmc, orc, batch, k, n):
     assert_f16_path(values(y), (g / (1 + torch.exp(-g)) * u).cpu().numpy(), what=f"{batch}x{k}x{n}")
 
 
+@pytest.mark.parametrize("batch,k,n", [(2, 520, 4096), (7, 4104, 5003), (16, 1160, 9000),
+                                       (30, 4104, 5003), (24, 520, 33000), (1, 4096, 4096)])
+def test_the_default_configuration_names_the_default(tmc, orc, batch, k, n):
+    """tmc_gemv_default_config's result gives the default's bits; so does
+    tmc_skinny_gemm_f16_mfma above batch 1."""
+    import torch
+    x = dev_f16(orc.f16(normal(4031 + batch, (batch, k))))
+    w, wu = (torch.empty((n, k), dtype=torch.float16, device="cuda") for _ in range(2))
+    tmc.fill_normal(w, 4032, 0.0, 0.02)
+    tmc.fill_normal(wu, 4033, 0.0, 0.02)
+    y, z, s = (torch.full((batch, n), float("nan"), device="cuda") for _ in range(3))
+    tmc.gemv(x, w, y)
+    tmc.gemv_config(x, w, z, tmc.default_config(batch, k, n))
+    assert torch.equal(y, z)
+    if batch > 1:
+        tmc.skinny_gemm(x, w, s)
+        assert torch.equal(y, s)
+    y, z = (torch.full((batch, n), float("nan"), dtype=torch.float16, device="cuda")
+            for _ in range(2))
+    tmc.gate_up_silu(x, w, wu, y)
+    tmc.gate_up_silu_config(x, w, wu, z, tmc.default_config(batch, k, n, True))
+    assert torch.equal(y, z)
+
+
 @pytest.mark.parametrize("cfg", [(3, 1, 4, 16), (3, 2, 4, 8), (3, 4, 2, 9), (3, 4, 1, 16),
                                  (3, 2, 1, 1)])
 def test_chosen_row_tiles_match_the_default(tmc, orc, cfg):
