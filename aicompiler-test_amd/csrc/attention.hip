@@ -881,6 +881,8 @@ __device__ __forceinline__ void consume_step_pvm(const AttnParams& p, const KvSt
 // marked slot leaves the output untouched) and resets the counter.  No
 // block waits for another and no cache writeback or invalidate is needed:
 // every shared word is written and read with agent-scope operations.
+constexpr bool merges_in_kernel(int d, int group) { return d == 128 && group <= 4; }
+
 template <int D, int GROUP, bool PAGED, int WAVES>
 __device__ void merge_if_last(const AttnParams& p, int b, int kvh, int nsplit) {
   __shared__ int s_last;
@@ -1118,7 +1120,8 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnParams p) 
   __syncthreads();
   finish_split<D, GROUP, PAGED, WAVES>(p, b, kvh, split, nsplit, bad, s_m, s_l, s_o);
   if constexpr (TL) timeline_put<TL>(6, shader_clock());
-  if (nsplit > 1 && p.arrivals) merge_if_last<D, GROUP, PAGED, WAVES>(p, b, kvh, nsplit);
+  if constexpr (merges_in_kernel(D, GROUP))
+    if (nsplit > 1 && p.arrivals) merge_if_last<D, GROUP, PAGED, WAVES>(p, b, kvh, nsplit);
   if constexpr (TL) {
     timeline_put<TL>(7, shader_clock());
     timeline_put<TL>(1, __builtin_amdgcn_s_memrealtime());
@@ -1131,7 +1134,7 @@ int launch_group(const AttnParams& params, int batch, hipStream_t stream) {
 #if TMC_ATTN_MERGE_LAUNCH
   p.arrivals = nullptr;  // build switch: every split merge in its own launch
 #endif
-  if (D != 128 || GROUP > 4) p.arrivals = nullptr;  // merge launch (see merge_if_last)
+  if (!merges_in_kernel(D, GROUP)) p.arrivals = nullptr;  // merge launch (see merge_if_last)
   const dim3 grid((unsigned)p.kv_heads, (unsigned)p.max_splits, (unsigned)batch);
 #define TMC_ATTN(MODE, WAVES)                                                                    \
   hipLaunchKernelGGL((attn_mfma_kernel<D, GROUP, MODE, WAVES>), grid, dim3(WAVES * kWave), 0,    \
