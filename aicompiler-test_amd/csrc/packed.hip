@@ -417,9 +417,14 @@ int row_tiles(int64_t batch, int64_t k, int mats, const PackedForm& form) {
 // against three: q.k.v (768 tiles) 21.6 / 29.7 / 34.0 against 20.1 / 22.6 /
 // 24.4 us, gate/up (688 pairs) 34.3 / 40.2 / 44.3 against 32.3 / 35.8 / 38.5,
 // LM head (2000) 51 / 71 / 85 against 46 / 55 / 60; two or four tiles were
-// slower than three on each.
-int column_tiles(int mt, int64_t n, int mats) {
-  if (mt == 1) return 1;
+// slower than three on each.  Three tiles' sums meet in LDS one after the
+// other, which takes K tiles of 128 to pay for: one a wave with one matrix,
+// two with two.  One tile against three, 24 / 48 / 64 rows: LM head K 512 11.1
+// / 14.0 / 17.4 against 10.5 / 15.9 / 17.5, K 1024 16.7 / 21.5 / 26.7 against
+// 15.9 / 20.0 / 22.4; gate/up K 1024 12.1 / 15.5 / 17.6 against 13.9 / 16.4 /
+// 17.6, K 2048 21.5 / 25.9 / 28.5 against 20.6 / 23.5 / 25.1.
+int column_tiles(int mt, int64_t k, int64_t n, int mats) {
+  if (mt == 1 || k < 1024 * mats) return 1;
   const double tiles = (double)((n + 15) / 16);
   const double one = tiles / 256.0 * (mt + mats);
   const double three = std::ceil(tiles / 3.0 / 256.0) * (mt + 3 * mats);
@@ -438,7 +443,7 @@ int run_packed(const half_t* x, const half_t* p0, const half_t* p1, OutT* y, int
   for (int64_t r0 = 0; r0 < batch; r0 += 16 * tiles) {
     const int rows = (int)std::min<int64_t>(16 * tiles, batch - r0);
     const int mt = (rows + 15) / 16;
-    const int nt = FUSE == kPackedResidual || form.chosen ? 1 : column_tiles(mt, n, MATS);
+    const int nt = FUSE == kPackedResidual || form.chosen ? 1 : column_tiles(mt, k, n, MATS);
     // of this pass alone: the last one may hold fewer row tiles, and then one
     // column tile, whose norm form is built for kPackedNormWaves waves
     const int waves = nt > 1 ? 8 : form.ks;

@@ -51,12 +51,13 @@ def test_row_tiles_equal_single_passes(tmc, orc, torch, batch, layout, k, n, ks)
         assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("batch,n", [(17, 12288), (33, 8208), (49, 8217), (64, 12300)])
-def test_three_column_tiles_match_fp64(tmc, orc, torch, batch, n):
-    """Wide outputs (three 16-column tiles per block, the last block short):
-    the fp32 projection within the fp32 rule of 64-bit sums of the same fp16
-    products, and the token-only LM head's tokens from the same logits."""
-    k = 1184
+@pytest.mark.parametrize("batch,n,k", [(17, 12288, 1184), (33, 8208, 1184), (49, 8217, 1184),
+                                       (64, 12300, 1184), (48, 12288, 1024), (48, 12288, 1016)])
+def test_three_column_tiles_match_fp64(tmc, orc, torch, batch, n, k):
+    """Wide outputs (three 16-column tiles per block from K 1024 on, the last
+    block short): the fp32 projection within the fp32 rule of 64-bit sums of
+    the same fp16 products, and the token-only LM head's tokens from the same
+    logits."""
     x = dev_f16(orc.f16(normal(2011 + batch, (batch, k))))
     gamma = dev_f16(orc.f16(uniform(2012, (k,), 0.5, 1.5)))
     w = dev_f16(orc.f16(normal(2013, (n, k), 0.02)))
@@ -83,7 +84,7 @@ def test_three_column_tiles_match_fp64(tmc, orc, torch, batch, n):
 def test_gated_rows_match_fp64(tmc, orc, torch, batch, n):
     """Gate/up + SiLU*Mul with the folded norm, packed output, at one and
     three tile pairs per block."""
-    k = 1184
+    k = 2088
     x = dev_f16(orc.f16(normal(2021 + batch, (batch, k))))
     one = dev_f16(orc.f16(np.ones(k, np.float32)))
     wg = dev_f16(orc.f16(normal(2022, (n, k), 0.02)))
@@ -103,7 +104,7 @@ def test_gated_rows_match_fp64(tmc, orc, torch, batch, n):
 def test_qkv_rope_rows_equal_unfused(tmc, orc, torch, batch, qh):
     """RoPE + append in the epilogue of several row (and column) tiles writes
     the bits of the packed GEMM followed by the append kernel."""
-    kvh, d, hidden, cap, p = qh, 64, 512, 64, 16
+    kvh, d, hidden, cap, p = qh, 64, 1032, 64, 16
     mp, width = cap // p, 3 * qh * 64
     rng = np.random.default_rng(2031)
     w = tmc.pack_weights(dev_f16(orc.f16(normal(2032, (width, hidden), 0.05))))
@@ -141,7 +142,7 @@ def _norm_ref(x, w, gamma):
 def test_norm_remainder_rows_match_fp64(tmc, orc, torch, batch, n):
     """Folded norm, a last pass of at most 16 rows after 64-row passes with
     three column tiles: logits and the token-only head's tokens."""
-    k = 264
+    k = 1096
     x = dev_f16(orc.f16(normal(2041 + batch, (batch, k))))
     gamma = dev_f16(orc.f16(uniform(2042, (k,), 0.5, 1.5)))
     w = dev_f16(orc.f16(normal(2043, (n, k), 0.02)))
@@ -161,7 +162,7 @@ def test_norm_remainder_rows_match_fp64(tmc, orc, torch, batch, n):
 def test_gated_remainder_rows_match_fp64(tmc, orc, torch, batch, n):
     """Gate/up: last passes of one to three row tiles with one column tile
     after passes with three."""
-    k = 264
+    k = 2056
     x = dev_f16(orc.f16(normal(2051 + batch, (batch, k))))
     one = dev_f16(orc.f16(np.ones(k, np.float32)))
     wg, wu = (dev_f16(orc.f16(normal(s, (n, k), 0.02))) for s in (2052, 2053))
@@ -178,7 +179,7 @@ def test_gated_remainder_rows_match_fp64(tmc, orc, torch, batch, n):
 def test_norm_qkv_remainder_rows_equal_their_own_call(tmc, orc, torch, batch):
     """Fused q.k.v of 12288 columns: the 64-row pass and the remainder write
     the bits of calls of their own, K/V pages included."""
-    qh, d, hidden, cap, p = 32, 128, 264, 64, 16
+    qh, d, hidden, cap, p = 32, 128, 1096, 64, 16
     mp, width = cap // p, 3 * qh * d
     rng = np.random.default_rng(2061)
     one = dev_f16(orc.f16(np.ones(hidden, np.float32)))
