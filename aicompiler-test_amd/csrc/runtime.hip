@@ -1637,12 +1637,15 @@ extern "C" int tmc_seq_create(tmc_runtime* rt, tmc_exec* const* steps, size_t n,
 namespace {
 // One replay of the sequence on its runtime's stream: the graph, or the
 // eager steps in order (stops at the first failing launch).  While the stream
-// is being captured a graph is launched as a graph.  The lock is held for both:
+// is being captured a graph is launched as a graph, and so is one that finds
+// an earlier error of the calling thread unread: a step's launch check would
+// take that error for its own and stop the replay.  The lock is held for both:
 // the runtime queues a graph's kernels one by one, and another thread's work
 // came between them (two threads replaying through one scratch buffer).
 int replay(tmc_seq* seq) {
   const std::lock_guard<std::mutex> lock(seq->rt->order);
-  if (seq->exec && (seq->eager.empty() || stream_captured(seq->rt)))
+  if (seq->exec && (seq->eager.empty() || hipPeekAtLastError() != hipSuccess ||
+                    stream_captured(seq->rt)))
     return hip_ok(hipGraphLaunch(seq->exec, seq->rt->stream), "graph launch");
   for (const auto& [launch, ctx] : seq->eager)
     if (launch(ctx)) return 1;

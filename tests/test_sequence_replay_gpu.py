@@ -82,6 +82,28 @@ def _run_threads(bodies):
         t.join()
 
 
+@pytest.mark.parametrize("steps", [1, 2, 6, 7])
+def test_an_unread_error_of_the_thread_is_not_the_replays(tmc, steps):
+    """A HIP call that the program itself made and that failed (a device that
+    does not exist), its error not yet read, does not stop a replay."""
+    import ctypes
+    import torch
+    rt = tmc.Runtime()
+    bufs, seq, _ = _chain(tmc, rt, torch, steps)
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    bufs[0].fill_(1.5)
+    torch.cuda.synchronize()
+    try:
+        assert hip.hipSetDevice(9999) != 0
+        seq.launch()
+    finally:
+        hip.hipGetLastError()
+    torch.cuda.synchronize()
+    rt_done = rt.wrap(bufs[-1]).read()  # after the replay, on its stream
+    assert bool((rt_done == 1.5 * 2.0 ** steps).all())
+
+
 @pytest.mark.parametrize("pairs", [1, 3, 5])
 def test_a_read_sees_whole_replays(tmc, pairs):
     """A buffer read from another thread falls before or after a replay."""
