@@ -83,6 +83,7 @@ def _declare(l):
         "tmc_prefill_attention_rows_f16": (i32, [vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i64,
                                                  i64, i64, i64, i64, i64, i64, i64, vp]),
         "tmc_gemm_rows_workspace_bytes": (sz, []),
+        "tmc_gemm_rows_plan": (i32, [i64, i64, i64, sz, vp]),
         "tmc_gemm_rows_f16": (i32, [vp, vp, vp, i32, i64, i64, i64, vp, sz, vp]),
         "tmc_gemm_mfma_f16": (i32, [vp, vp, vp, i32, i64, i64, i64, vp]),
         "tmc_prefill_attention_f16": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64,
@@ -619,6 +620,13 @@ def prefill_attention_rows(q, k_pool, v_pool, valid_lengths, tables, row_table, 
 
 def gemm_rows_workspace_bytes() -> int:
     return int(lib().tmc_gemm_rows_workspace_bytes())
+
+
+def gemm_rows_plan(m, k, n, workspace_bytes=0) -> tuple:
+    """(tile rows, tile columns, stages in LDS, splits of K) of gemm_rows."""
+    out = (C.c_int32 * 4)()
+    check(lib().tmc_gemm_rows_plan(m, k, n, workspace_bytes, out), "tmc_gemm_rows_plan")
+    return tuple(out)
 
 
 def gemm_rows(x, w, y, workspace=None, stream=None):

@@ -259,7 +259,6 @@ int launch_plan(const TilePlan& plan, const half_t* x, const half_t* w, OutT* y,
     TMC_TILE(2, 2, 4, 4, 1, 4);
   }
   switch (plan.bn) {
-  case 128: TMC_TILE(4, 2, 4, 4, 2, 2);
   case 160: TMC_TILE(4, 2, 4, 5, 2, 2);
   case 192: TMC_TILE(4, 2, 4, 6, 2, 2);
   default: TMC_TILE(2, 4, 8, 4, 2, 2);
@@ -274,7 +273,9 @@ int launch_plan(const TilePlan& plan, const half_t* x, const half_t* w, OutT* y,
 // further rounds.  A split adds the reduction: 3.9 us and 2.8 us per million
 // partials.  The figures are a fit to 2000 launches (40 shapes, m 16-2048, k
 // 1000-11008, n 2048-12288, every tile and split); its choices are within 1%
-// of the best in the middle and 24% at worst, and 1.02 to 1.75 times as fast
+// of the best in the middle and 24% at worst (a 256 x 128 tile takes what two
+// 128 x 128 tiles on one CU take, 1.024 us, and is never chosen: not built),
+// and 1.02 to 1.75 times as fast
 // as 128 x 128 and 256 x 256 tiles chosen by their count (1.31 in the mean):
 // 2048 x 4096 x 12288 240 -> 184 us (256 x 192: two whole rounds where 256 x
 // 256 leaves half of the second idle), 1024 x 4096 x 4096 57 -> 40 (four
@@ -286,8 +287,7 @@ TilePlan tile_plan(int64_t m, int64_t k, int64_t n, size_t workspace_bytes) {
   };
   static constexpr Tile kTiles[] = {
       {64, 128, 4, 0.405, 0},  {128, 128, 2, 0.787, 1.024}, {128, 128, 4, 0.571, 0},
-      {256, 128, 2, 1.024, 0}, {256, 160, 2, 1.108, 0},     {256, 192, 2, 1.236, 0},
-      {256, 256, 2, 1.497, 0}};
+      {256, 160, 2, 1.108, 0}, {256, 192, 2, 1.236, 0},     {256, 256, 2, 1.497, 0}};
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
   TilePlan best{256, 256, 2, 1};
   double least = 1e30;
@@ -313,6 +313,11 @@ TilePlan tile_plan(int64_t m, int64_t k, int64_t n, size_t workspace_bytes) {
   return best;
 }
 
+// k per split, in whole stages
+int64_t split_length(int64_t k, int splits) {
+  return ((k + splits - 1) / splits + kStageK - 1) / kStageK * kStageK;
+}
+
 int launch_gemm(const half_t* x, const half_t* w, void* y, int out_dtype, int64_t m, int64_t k,
                 int64_t n, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   const uint64_t xb = (uint64_t)m * k * 2, wb = (uint64_t)n * k * 2;
@@ -321,8 +326,7 @@ int launch_gemm(const half_t* x, const half_t* w, void* y, int out_dtype, int64_
   TMC_REQUIRE(k % 8 == 0, "Prompt GEMM: k must be a multiple of 8.");
   TMC_REQUIRE(aligned16(x) && aligned16(w), "Prompt GEMM: x and w must be 16-byte aligned.");
   const TilePlan plan = tile_plan(m, k, n, workspace ? workspace_bytes : 0);
-  // k per split, in whole stages
-  const int k_chunk = (int)(((k + plan.splits - 1) / plan.splits + kStageK - 1) / kStageK * kStageK);
+  const int k_chunk = (int)split_length(k, plan.splits);
   const int used = (int)((k + k_chunk - 1) / k_chunk);
   if (used > 1) {
     float* partial = static_cast<float*>(workspace);
@@ -350,6 +354,20 @@ extern "C" int tmc_gemm_mfma_f16(const void* x, const void* weight, void* y, int
               "Prompt GEMM: invalid shape.");
   return launch_gemm(static_cast<const half_t*>(x), static_cast<const half_t*>(weight), y,
                         out_dtype, m, k, n, nullptr, 0, as_stream(stream));
+}
+
+extern "C" int tmc_gemm_rows_plan(int64_t m, int64_t k, int64_t n, size_t workspace_bytes,
+                                  int32_t out[4]) {
+  TMC_REQUIRE(out, "Prompt GEMM: null plan.");
+  TMC_REQUIRE(m > 0 && k > 0 && n > 0 && m < (1LL << 31) && k < (1LL << 31) && n < (1LL << 31),
+              "Prompt GEMM: invalid shape.");
+  const TilePlan plan = tile_plan(m, k, n, workspace_bytes);
+  const int64_t length = split_length(k, plan.splits);
+  out[0] = plan.bm;
+  out[1] = plan.bn;
+  out[2] = plan.stages;
+  out[3] = (int32_t)((k + length - 1) / length);
+  return 0;
 }
 
 extern "C" size_t tmc_gemm_rows_workspace_bytes(void) { return (size_t)32 << 20; }

@@ -683,9 +683,9 @@ int tmc_prefill_rope_append_rows(const void *qkv, const float *cosine, const flo
 /* emitTiledGEMM (DecodeGEMVMetalEmitter.cpp:134-169), the prefill linear
  * layer: y[m, n] = x[m, k] weight[n, k]^T, fp16 inputs, fp32 accumulation,
  * y fp16 or fp32 (out_dtype), all row-major, on the hand-written gfx950 MFMA
- * GEMM (v_mfma_f32_16x16x32_f16, 128 x 128 output tiles per 256-thread
- * workgroup; k a multiple of 8, x and weight 16-byte aligned and each below
- * 4 GiB).  When the output tiles alone would leave CUs idle and the
+ * GEMM (v_mfma_f32_16x16x32_f16, output tiles of 64 x 128 to 256 x 256 by
+ * shape, see tmc_gemm_rows_plan; k a multiple of 8, x and weight 16-byte
+ * aligned and each below 4 GiB).  When the output tiles alone would leave CUs idle and the
  * workspace holds the fp32 partials, K is split over several workgroups and
  * a second launch adds the partials in split order.  workspace may be NULL
  * with workspace_bytes 0 (no split); tmc_gemm_rows_workspace_bytes() is the
@@ -696,6 +696,9 @@ size_t tmc_gemm_rows_workspace_bytes(void);
 /* tmc_gemm_rows_f16 without a workspace (never splits K). */
 int tmc_gemm_mfma_f16(const void *x, const void *weight, void *y, int out_dtype, int64_t m,
                       int64_t k, int64_t n, void *stream);
+/* The launch tmc_gemm_rows_f16 chooses for a shape and workspace size: tile
+ * rows, tile columns, stages of 64 k in LDS, splits of K.  Host only. */
+int tmc_gemm_rows_plan(int64_t m, int64_t k, int64_t n, size_t workspace_bytes, int32_t out[4]);
 int tmc_gemm_rows_f16(const void *x, const void *weight, void *y, int out_dtype, int64_t m,
                       int64_t k, int64_t n, void *workspace, size_t workspace_bytes,
                       void *stream);
