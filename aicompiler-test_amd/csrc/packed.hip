@@ -398,8 +398,10 @@ int lm_head_unroll(int64_t batch) { return batch > 8 ? 1 : 4; }
 // packed activations, weights beyond the caches: gate/up 121 -> 44 us, q.k.v
 // 73 -> 34, down 69 -> 30, o 31 -> 13, against floors of 28, 16, 14 and 6).
 // What bounds a launch from there is not HBM but the activation fragments,
-// which every output tile re-reads from L2 (about 15 TB/s over the chip).
-// The two-matrix form holds at most 8 waves' partial sums in 64 KiB of LDS.
+// which every output tile re-reads from L2 (down at 50 rows: 12.7 TB/s of L2
+// requests over the chip, three quarters of them hits).
+// The two-matrix form holds at most 8 waves' partial sums in LDS (64 KiB, and
+// 2 KiB of squares with the folded norm).
 // A caller's unroll bounds the tiles whose loads it holds in registers: four
 // row tiles at 1, two at 2, one at 4.
 int row_tiles(int64_t batch, int64_t k, int mats, const PackedForm& form) {

@@ -16,7 +16,8 @@ Subcommands over the rocpd SQLite databases rocprofv3 writes:
            kernel that issues MFMA, with achieved TFLOP/s from the trace;
   stalls   issue and stall counters (SQ wave / wait / issue cycles, VMEM
            latency, occupancy, TA busy, TCP-to-L2 request latency, address
-           translation) per dispatch of chosen kernels, with per-wave ratios;
+           translation, LDS conflicts, MFMA use, L2 requests) per dispatch of
+           chosen kernels, with per-wave ratios;
   c4       the C4 record: the paged attention kernel and the gather probe
            over the same bytes, their traffic rows (from `table --json`) and
            stall rows (from `stalls --json`) side by side.
@@ -263,15 +264,18 @@ STALL_COUNTERS = (
     "VmemLatency", "MeanOccupancyPerCU", "MeanOccupancyPerActiveCU",
     "TA_TA_BUSY_sum", "TA_ADDR_STALLED_BY_TC_CYCLES_sum",
     "TCP_TCC_READ_REQ_LATENCY_sum", "TCP_TCC_READ_REQ_sum",
-    "TCP_UTCL1_TRANSLATION_MISS_sum", "TCP_UTCL1_TRANSLATION_HIT_sum")
+    "TCP_UTCL1_TRANSLATION_MISS_sum", "TCP_UTCL1_TRANSLATION_HIT_sum",
+    "SQ_LDS_BANK_CONFLICT", "SQ_LDS_IDX_ACTIVE", "MfmaUtil", "TCC_HIT_sum", "TCC_MISS_sum")
 
 
 def stall_table(dbs: list, trace_db: str, kernels: list, min_calls: int) -> list:
     """Mean of every stall counter per (kernel, grid) whose short name contains
     one of `kernels`, merged over the pass databases, plus per-wave ratios:
     SQ_WAIT_ANY / SQ_WAVES (cycles a wave spends waiting on a counter),
-    SQ_ACTIVE_INST_ANY / SQ_WAVES (cycles it issues), and the average
-    TCP-to-L2 read latency (TCP_TCC_READ_REQ_LATENCY / TCP_TCC_READ_REQ)."""
+    SQ_ACTIVE_INST_ANY / SQ_WAVES (cycles it issues), the average TCP-to-L2
+    read latency (TCP_TCC_READ_REQ_LATENCY / TCP_TCC_READ_REQ), bank-conflict
+    cycles over the LDS's active cycles, and L2 requests of 128 bytes over the
+    trace's time."""
     merged = collections.defaultdict(dict)
     for db in dbs:
         for key, d in _per_kernel(db, STALL_COUNTERS).items():
@@ -304,6 +308,13 @@ def stall_table(dbs: list, trace_db: str, kernels: list, min_calls: int) -> list
         miss = counters.get("TCP_UTCL1_TRANSLATION_MISS_sum")
         if hit is not None and miss is not None and hit + miss:
             row["utcl1_miss_pct"] = round(100.0 * miss / (hit + miss), 2)
+        if counters.get("SQ_LDS_IDX_ACTIVE"):
+            row["lds_conflict_pct"] = round(100.0 * counters.get("SQ_LDS_BANK_CONFLICT", 0.0) /
+                                            counters["SQ_LDS_IDX_ACTIVE"], 2)
+        requests = counters.get("TCC_HIT_sum", 0.0) + counters.get("TCC_MISS_sum", 0.0)
+        if requests:
+            row["l2_hit_pct"] = round(100.0 * counters.get("TCC_HIT_sum", 0.0) / requests, 2)
+            row["l2_tbps"] = round(requests * 128.0 / (row["avg_us"] * 1e6), 2)
         rows.append(row)
     rows.sort(key=lambda x: -x["avg_us"] * x["calls"])
     return rows
@@ -329,7 +340,7 @@ def c4_record(traffic_json: str, stalls_json: str, command: str) -> dict:
         return max(found, key=lambda r: r["calls"] * r["avg_us"])
 
     out = {"workload": C4_WORKLOAD, "command": command, "scales": traffic_rows["scales"]}
-    for key, name in (("attention_kernel", "attn_mfma_kernel<4, 1, 4>"),
+    for key, name in (("attention_kernel", "attn_mfma_kernel<128, 4, 1, 4>"),
                       ("gather_probe", "gather_probe_kernel")):
         out[key] = {"traffic": pick(traffic_rows["kernels"], name),
                     "stalls": pick(stall_rows, name)}
