@@ -436,8 +436,10 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
   constexpr int CH = D / 8, RPI = kWave / CH, QI = 16 / RPI;  // chunks a row, rows a load, loads
   __shared__ __attribute__((aligned(16))) half_t s_even[2 * BLOCK * D];  // K rows, V rows
   __shared__ __attribute__((aligned(16))) half_t s_odd[2 * BLOCK * D];
-  __shared__ int s_bounds[2];
   extern __shared__ int s_table[];
+  // read before the first load into that buffer: 64 KiB a 4-wave block at D =
+  // 128, so that two of them fit a CU beside tables of 16 KiB
+  int* s_bounds = reinterpret_cast<int*>(s_odd);
   typedef __attribute__((address_space(3))) void lds_void;
 
   const int id = blockIdx.x;
@@ -820,7 +822,12 @@ extern "C" int tmc_prefill_attention_rows_f16(const void* q, const void* key_poo
     // more blocks than CUs two 4-wave blocks share a CU and two groups win
     // (2048 tokens MHA 74 against 83), and below about 500 positions the
     // longer hand-over costs more than it saves (200 tokens 9.2 against 10.6).
-    const bool four = grid.x <= 256 && page_size * max_pages > 1024;
+    // Where tables over 16 KiB leave room for one 4-wave block a CU, four groups
+    // run there too.  2048 tokens at 2000, 64 heads on 8, pages of one: table of
+    // 24 KiB 350 us with four groups, 453 with two (16-vector kernel 509), and
+    // of 16 KiB 290 us with two blocks a CU.
+    const bool pairs = head_dim == 64 || 2 * (64 * 1024 + table_lds) <= 160 * 1024;
+    const bool four = page_size * max_pages > 1024 && (grid.x <= 256 || !pairs);
 #define TMC_PT_LAUNCH(DIM, PG) \
   hipLaunchKernelGGL((prefill_tile_kernel<DIM, PG>), grid, dim3(2 * PG * kWave), table_lds, s, p)
     if (head_dim == 128) {
