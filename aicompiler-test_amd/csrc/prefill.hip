@@ -411,8 +411,10 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
 // MI355X, against the 16-vector kernel: 512 tokens at 3584 (GQA 4) 105 -> 56
 // us, 2048 tokens (MHA) 96 -> 74 (470 TFLOP/s), head dim 64, 1024 at 1024
 // 50 -> 31.  Error against 64 bits over contexts of 2000 to 4096: 2.75e-4 of
-// the rms, 2.82e-4 before (2.07e-4 of it the output's rounding).  What bounds it now is the softmax's VALU work beside the MFMAs,
-// and for few blocks the latency of one block's loads.
+// the rms, 2.82e-4 before (2.07e-4 of it the output's rounding).
+// What bounds it now: scores, softmax and PV run one after the other in a wave,
+// and two waves a SIMD leave the matrix cores 21% busy (512 tokens at 3584); for
+// few blocks the latency of one block's loads.
 constexpr size_t kPtTable = 28 * 1024;  // block-table bytes beside 128 KiB of buffers
 
 // Maximum over the four lane groups of a wave (lanes l, l + 16, l + 32, l + 48),
@@ -503,12 +505,13 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
   const long bad_from = (long)s_bounds[1] * p.page_size;  // positions at/after: absent page
 
   const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  h8 qb[2][KS];
+  h8 qb[2][KS];  // a group past the attended positions needs none
 #pragma unroll
   for (int v = 0; v < 2; ++v) {
     const half_t* qrow = p.q + ((size_t)token[v] * p.q_heads + head[v]) * D;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qb[v][s] = len[v] > 0 ? load_h8(qrow + 32 * s + 8 * g) : zero;
+    for (int s = 0; s < KS; ++s)
+      qb[v][s] = len[v] > 0 && 32 * ph < end ? load_h8(qrow + 32 * s + 8 * g) : zero;
   }
 
   // stage loads: load q of this wave moves rows 16 wave + RPI q ... of the
@@ -517,6 +520,8 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
   const __amdgpu_buffer_rsrc_t rv = buffer_resource(p.v, p.pool_bytes);
   const int slot = lane % CH;
   auto load = [&](int base, half_t* buf) {
+    // a group loads the rows that it alone reads: none past the attended ones
+    if (base + 32 * ph >= end) return;
     int page[QI], row[QI];
     if (p.page_shift >= 0) {
 #pragma unroll
@@ -681,9 +686,10 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     Frags f;
-    read(now, f);
-    if (base + BLOCK < end) load(base + BLOCK, then);
-    if (base + 32 * ph < wave_max) compute(base, f);
+    const bool mine = base + 32 * ph < wave_max;
+    if (mine) read(now, f);
+    load(base + BLOCK, then);
+    if (mine) compute(base, f);
   };
   load(0, s_even);
   for (int base = 0; base < end; base += 2 * BLOCK) {
@@ -691,55 +697,76 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
     if (base + BLOCK < end) step(base + BLOCK, s_odd, s_even);
   }
 
-  // the position groups meet: the others hand group 0 their sums through LDS
-  __syncthreads();
+  // The position groups meet: group 0 finishes the first vector tile, group 1
+  // the second, and the others hand them their sums through LDS.  Groups past
+  // the attended positions loaded nothing and hand nothing, and a lone group
+  // meets nobody.  Prompts from position 0 of a 4096-position cache, GQA 4, 1 /
+  // 16 / 64 / 200 tokens: 5.1 / 6.6 / 7.5 / 10.8 us, where all four groups
+  // handed both tiles to group 0 6.7 / 9.2 / 9.3 / 10.9 (16-vector kernel 5.1 /
+  // 6.3 / 6.5 / 10.8).
+  const int groups = min(PG, (end + 31) / 32);
   constexpr int kHand = (2 + 4 * DT) * kWave;  // floats a vector tile hands over
   static_assert((PG - 1) * 2 * kHand * 4 <= 2 * BLOCK * D * 2, "the handed sums fit one buffer");
   float* hand = reinterpret_cast<float*>(vh ? s_odd : s_even) + lane;
-  if (ph > 0) {
-#pragma unroll
-    for (int v = 0; v < 2; ++v) {
-      float* at = hand + (2 * (ph - 1) + v) * kHand;
-      at[0] = m[v];
-      at[kWave] = lsum[v][0];
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) at[(2 + 4 * t + r) * kWave] = o[v][t][r];
-    }
-  }
-  __syncthreads();
-  if (ph > 0) return;
-#pragma unroll
-  for (int v = 0; v < 2; ++v) {
-    if (len[v] <= 0 || len[v] > bad_from) continue;
-    float top = m[v];
-#pragma unroll
-    for (int q = 0; q < PG - 1; ++q) top = fmaxf(top, hand[(2 * q + v) * kHand]);
-    // a group without positions of this query holds -inf and zeros
-    const float own = m[v] == -INFINITY ? 0.0f : fast_exp2(m[v] - top);
-    float sum = own * lsum[v][0];
-#pragma unroll
-    for (int t = 0; t < DT; ++t) o[v][t] *= own;
-#pragma unroll
-    for (int q = 0; q < PG - 1; ++q) {
-      const float* at = hand + (2 * q + v) * kHand;
-      const float other = at[0];
-      const float scale = other == -INFINITY ? 0.0f : fast_exp2(other - top);
-      sum += scale * at[kWave];
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[v][t][r] += scale * at[(2 + 4 * t + r) * kWave];
-    }
+  // tile v's sums of group q, which does not finish it
+  auto handed = [&](int v, int q) { return hand + ((PG - 1) * v + q - (q > v ? 1 : 0)) * kHand; };
+  auto finish = [&](int v, float sum, const f4 (&total)[DT]) {
     const float inv = 1.0f / sum;
     half_t* orow = p.out + ((size_t)token[v] * p.q_heads + head[v]) * D;
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-      const h4 val = {(half_t)(o[v][t][0] * inv), (half_t)(o[v][t][1] * inv),
-                      (half_t)(o[v][t][2] * inv), (half_t)(o[v][t][3] * inv)};
+      const h4 val = {(half_t)(total[t][0] * inv), (half_t)(total[t][1] * inv),
+                      (half_t)(total[t][2] * inv), (half_t)(total[t][3] * inv)};
       *reinterpret_cast<h4*>(orow + 16 * t + 4 * g) = val;
     }
+  };
+  if (groups == 1) {
+    if (ph > 0) return;
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      if (len[v] > 0 && len[v] <= bad_from) finish(v, lsum[v][0], o[v]);
+    return;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    if (ph == v || ph >= groups) continue;
+    float* at = handed(v, ph);
+    at[0] = m[v];
+    at[kWave] = lsum[v][0];
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) at[(2 + 4 * t + r) * kWave] = o[v][t][r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    if (ph != v || len[v] <= 0 || len[v] > bad_from) continue;
+    float top = m[v];
+#pragma unroll
+    for (int q = 0; q < PG; ++q)
+      if (q != v && q < groups) top = fmaxf(top, handed(v, q)[0]);
+    // in group order; a group without positions of this query holds -inf and zeros
+    float sum = 0.0f;
+    f4 total[DT];
+#pragma unroll
+    for (int q = 0; q < PG; ++q) {
+      if (q >= groups) break;
+      const float* at = handed(v, q == v ? 1 - v : q);
+      const float high = q == v ? m[v] : at[0];
+      const float scale = high == -INFINITY ? 0.0f : fast_exp2(high - top);
+      const float part = q == v ? lsum[v][0] : at[kWave];
+      sum = q == 0 ? scale * part : sum + scale * part;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = q == v ? o[v][t][r] : at[(2 + 4 * t + r) * kWave];
+          total[t][r] = q == 0 ? scale * x : total[t][r] + scale * x;
+        }
+    }
+    finish(v, sum, total);
   }
 }
 
@@ -821,7 +848,8 @@ extern "C" int tmc_prefill_attention_rows_f16(const void* q, const void* key_poo
     // GQA 4: 56 us against 72 with two groups, 16 at 3000 43 against 56; with
     // more blocks than CUs two 4-wave blocks share a CU and two groups win
     // (2048 tokens MHA 74 against 83), and below about 500 positions the
-    // longer hand-over costs more than it saves (200 tokens 9.2 against 10.6).
+    // longer hand-over costs more than it saves (200 tokens, MHA 9.5 against
+    // 10.8).
     // Where tables over 16 KiB leave room for one 4-wave block a CU, four groups
     // run there too.  2048 tokens at 2000, 64 heads on 8, pages of one: table of
     // 24 KiB 350 us with four groups, 453 with two (16-vector kernel 509), and

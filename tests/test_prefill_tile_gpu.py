@@ -31,7 +31,13 @@ def _attend64(torch, q, k, v, start):
     (40, 8, 2, 64, 4, 100, 32000, 0, 1), (33, 8, 2, 64, 2, 75, 16000, 0, 30),
     (50, 8, 4, 64, 16, 70, 128, 5, 30), (50, 8, 4, 128, 12, 70, 132, 3, 1),
     (20, 4, 4, 128, 1, 30, 64, 1, 1), (600, 32, 32, 128, 1, 0, 4096, 0, 1),
-    (600, 32, 32, 128, 1, 40, 5000, 0, 1)])
+    (600, 32, 32, 128, 1, 40, 5000, 0, 1),
+    # one to four position groups with attended positions, of two and of four
+    (1, 8, 8, 128, 16, 0, 2048, 0, 1), (32, 8, 8, 128, 16, 0, 2048, 0, 30),
+    (64, 8, 2, 128, 16, 0, 2048, 0, 1), (65, 4, 4, 128, 16, 0, 2048, 0, 30),
+    (97, 8, 8, 64, 16, 0, 4096, 0, 1), (16, 64, 8, 64, 16, 0, 2048, 0, 1),
+    (31, 8, 1, 128, 16, 33, 2048, 0, 1), (33, 8, 2, 128, 16, 0, 512, 0, 1),
+    (64, 64, 8, 64, 16, 0, 512, 0, 30)])
 def test_prefill_tiles_match_fp64(tmc, rows, qh, kvh, d, p, start, capacity, pad, sharp):
     """pad > 0 moves the heads of a page apart by an odd element count; these,
     and tables past 28 KiB, run the staged-register kernel with the table in
