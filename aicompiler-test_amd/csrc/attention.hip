@@ -1265,17 +1265,27 @@ SplitPlan split_plan(int64_t head_dim, int64_t batch, int64_t q_heads, int64_t k
 // the workspace is sized for.  MI355X, random pages, VALU against MFMA: GQA 4
 // batch 24, 100-2000 positions 27.6 against 18.9 us, batch 64, 200-1500 41.0
 // against 30.7, batch 1 at 4000 12.3 against 9.9; GQA 8 batch 64, 100-2000
-// 62.1 against 24.5; one-split MHA batch 1 at 300 7.3 against 5.4, batch 8,
-// 100-900 12.9 against 10.9.  Elsewhere MHA and GQA 2 are as fast or faster
-// on VALU (batch 24 MHA, 50-250: 9.4 against 13.7; GQA 2 batch 64, 100-600
-// 27.0 against 27.2), and so are other page sizes (12: 27.9 against 28.6).
+// 62.1 against 24.5.  MHA and GQA 2 take one 16-wave block a row where the VALU
+// kernel would split it (caches rotated; paged, capacity 512 and 1024, batch 1,
+// 32 heads, at 200-500 8.3 against 6.4, 8 kv heads on 16 batch 8, 300-500 9.6
+// against 8.2, full rows of 1024 8.5 against 8.0-8.7; contiguous 512, batch 4,
+// at 500 8.8 against 6.7).  Where one VALU block covers the row anyway the 16
+// waves only cost (paged capacity 128 4.3 against 4.7, contiguous 256 at 250
+// 4.2 against 4.9), and so they do on few long contiguous rows, which walk two
+// or more steps a wave (1024, 32 rows at 500 6.5 against 6.1, at 1024 7.1
+// against 8.9; 48 rows 8.3 against 9.0, 64 9.0 against 9.2, 128 11.7 against
+// 10.0).  Elsewhere MHA and GQA 2 are as fast or faster on VALU (batch 24 MHA,
+// 50-250: 9.4 against 13.7; GQA 2 batch 64, 100-600 27.0 against 27.2), and so
+// are other page sizes (12: 27.9 against 28.6).
 SplitPlan launch_plan(int64_t head_dim, int64_t batch, int64_t q_heads, int64_t kv_heads,
-                      int64_t capacity, bool whole_rows) {
+                      int64_t capacity, bool whole_rows, bool paged) {
   const SplitPlan plan = split_plan(head_dim, batch, q_heads, kv_heads, capacity);
   if (head_dim != 64 || !whole_rows) return plan;
   if (q_heads / kv_heads > kWideMaxGroup)
     return {batch * kv_heads * capacity / 256 >= 1024 ? 2 * plan.chunk : plan.chunk, kWaves, false};
-  if (capacity <= kMfmaMaxChunk && batch * kv_heads <= kWideMaxRows)
+  const int64_t rows = batch * kv_heads;
+  if (capacity > plan.chunk && capacity <= kMfmaMaxChunk && rows <= kWideMaxRows &&
+      (paged || capacity <= 512 || rows >= 48))
     return {(int)((capacity + kMfmaStep - 1) / kMfmaStep * kMfmaStep), kWideWaves, false};
   return plan;
 }
@@ -1382,7 +1392,7 @@ extern "C" int tmc_decode_attention(const void* q, const void* key_cache, const 
     p.kv_bytes = bytes < kAbsent ? (unsigned)bytes : 0u;
   }
   const SplitPlan plan =
-      launch_plan(head_dim, batch, q_heads, kv_heads, capacity, p.kv_bytes != 0);
+      launch_plan(head_dim, batch, q_heads, kv_heads, capacity, p.kv_bytes != 0, false);
   p.chunk = plan.chunk;
   p.waves = plan.waves;
   p.valu = plan.valu;
@@ -1442,7 +1452,7 @@ int paged_attention_impl(const void* q, const void* key_pool, const void* value_
   }
   p.max_pages = (int)max_pages;
   const SplitPlan plan = launch_plan(head_dim, max_batch, q_heads, kv_heads, capacity,
-                                     p.kv_bytes != 0 && page_size % 16 == 0);
+                                     p.kv_bytes != 0 && page_size % 16 == 0, true);
   p.chunk = plan.chunk;
   p.waves = plan.waves;
   p.valu = plan.valu;

@@ -28,7 +28,10 @@ def _ref(torch, q, k, v):
     (16, 2, 16, [1, 255, 256, 257, 600, 1000], 1024, 1), (32, 8, 16, [2047, 5, 1300] * 8, 2048, 30),
     (8, 1, 48, [700, 47, 49, 95], 960, 30), (4, 4, 16, [1, 32, 511, 512, 513, 1023], 1024, 1),
     (8, 4, 32, [900, 3, 33], 1024, 30), (32, 32, 16, [300] * 9 + [1], 512, 1),
-    (8, 2, 12, [500, 11, 12, 13], 504, 1), (4, 4, 16, [1500, 20], 2048, 1)])
+    (8, 2, 12, [500, 11, 12, 13], 504, 1), (4, 4, 16, [1500, 20], 2048, 1),
+    # one VALU split; the first row lengths past it
+    (4, 4, 16, [1, 15, 127, 128], 128, 1), (8, 4, 16, [255, 256, 33], 256, 30),
+    (4, 4, 16, [256, 257, 272], 272, 1)])
 def test_paged_d64_matches_fp64(tmc, qh, kvh, p, lengths, capacity, sharp):
     import torch
     torch.manual_seed(qh * 100 + p)
@@ -68,7 +71,8 @@ def test_paged_d64_matches_fp64(tmc, qh, kvh, p, lengths, capacity, sharp):
 
 @pytest.mark.parametrize("b,qh,kvh,capacity,length", [
     (1, 8, 2, 2048, 2047), (1, 32, 8, 4096, 1025), (2, 8, 1, 512, 31), (1, 8, 8, 1024, 900),
-    (1, 4, 4, 2000, 1999),
+    (1, 4, 4, 2000, 1999), (1, 8, 8, 512, 511), (2, 8, 4, 257, 257), (1, 4, 4, 256, 256),
+    (2, 48, 24, 1024, 1023), (1, 47, 47, 1024, 513),  # 48 and 47 rows past 512 positions
     (64, 32, 32, 16384, 300)])  # 4 GiB a cache: past the buffer loads' range
 def test_contiguous_d64_matches_fp64(tmc, b, qh, kvh, capacity, length):
     import torch
