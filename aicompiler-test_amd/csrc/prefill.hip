@@ -686,10 +686,9 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     Frags f;
-    const bool mine = base + 32 * ph < wave_max;
-    if (mine) read(now, f);
+    read(now, f);
     load(base + BLOCK, then);
-    if (mine) compute(base, f);
+    if (base + 32 * ph < wave_max) compute(base, f);
   };
   load(0, s_even);
   for (int base = 0; base < end; base += 2 * BLOCK) {
@@ -701,7 +700,7 @@ __global__ __launch_bounds__(2 * PG * kWave, 2) void prefill_tile_kernel(Prefill
   // the second, and the others hand them their sums through LDS.  Groups past
   // the attended positions loaded nothing and hand nothing, and a lone group
   // meets nobody.  Prompts from position 0 of a 4096-position cache, GQA 4, 1 /
-  // 16 / 64 / 200 tokens: 5.1 / 6.6 / 7.5 / 10.8 us, where all four groups
+  // 16 / 64 / 200 tokens: 5.1 / 6.7 / 7.5 / 10.7 us, where all four groups
   // handed both tiles to group 0 6.7 / 9.2 / 9.3 / 10.9 (16-vector kernel 5.1 /
   // 6.3 / 6.5 / 10.8).
   const int groups = min(PG, (end + 31) / 32);
