@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kPaThreads) void prefill_attention_kernel(PrefillPa
 // 50 -> 31.  Error against 64 bits over contexts of 2000 to 4096: 2.75e-4 of
 // the rms, 2.82e-4 before (2.07e-4 of it the output's rounding).
 // What bounds it now: scores, softmax and PV run one after the other in a wave,
-// and two waves a SIMD leave the matrix cores 21% busy (512 tokens at 3584); for
+// and two waves a SIMD leave the matrix cores 20% busy (512 tokens at 3584); for
 // few blocks the latency of one block's loads.
 constexpr size_t kPtTable = 28 * 1024;  // block-table bytes beside 128 KiB of buffers
 
